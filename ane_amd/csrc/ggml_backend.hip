@@ -26,6 +26,7 @@
 #include "../../include/ggml-ane-hip.h"
 #include "common.hpp"
 #include "ggml_rows.hpp"
+#include "rmode_mul_mat.hpp"
 
 struct ane_ggml_backend {
     hipStream_t stream;
@@ -132,9 +133,15 @@ int mul_mat_rows(ane_ggml_backend* be, int type, uint32_t N, uint32_t K, uint32_
     if (g) {
         st = ane_hip_q8_0_mul_mat(N, K, T, xp, W, yp, ws, qws, be->stream);
     } else {
-        const auto gemv = type == ANE_GGML_TYPE_Q8_0 ? ane_hip_q8_0_gemv : ane_hip_q4_0_gemv;
-        for (uint32_t t = 0; t < T && st == ANE_OK; t++)
-            st = gemv(N, K, xp + (uint64_t)t * K, W, yp + (uint64_t)t * N, be->stream);
+        const bool q4 = type == ANE_GGML_TYPE_Q4_0;
+        st = T >= 2 ? rmode_mul_mat(q4, N, K, T, xp, W, yp, be->stream) : -1;
+        if (st == -1) {
+            // one token, or a shape that kernel does not take
+            const auto gemv = q4 ? ane_hip_q4_0_gemv : ane_hip_q8_0_gemv;
+            st = ANE_OK;
+            for (uint32_t t = 0; t < T && st == ANE_OK; t++)
+                st = gemv(N, K, xp + (uint64_t)t * K, W, yp + (uint64_t)t * N, be->stream);
+        }
     }
     if (st != ANE_OK) return st;
     if (!yc) {

@@ -64,7 +64,7 @@ enum ane_ggml_op {
 
 /* Q8_0 arithmetic of MUL_MAT: G quantizes each activation row per 32-block
  * and dots int8 x int8 (the default); R is the reference opcode 0x57's fp32
- * arithmetic (bytecode_interpreter.s:7010-7063), one launch per token. */
+ * arithmetic (bytecode_interpreter.s:7010-7063) for every token. */
 enum ane_ggml_q8_mode { ANE_GGML_Q8_G = 0, ANE_GGML_Q8_R = 1 };
 
 struct ane_ggml_tensor {
