@@ -13,8 +13,8 @@
 // [row][128 bytes] with the 16-byte chunk index XOR-swizzled by
 // (row ^ row>>3) & 7 so the ds_read_b128 of 16 consecutive rows (one LDS
 // cycle: 64 banks x 4 bytes) hits 16 distinct bank groups.  Large shapes use the 256 x 256 kernel of
-// gemm_i8_tile256.hip instead, and up to 128 rows the few-row kernel of
-// gemm_i8_skinny.hip.
+// gemm_i8_tile256.hip instead (128 x 128 below one 256-tile per CU), few rows
+// the kernel of gemm_i8_skinny.hip, both also on SMOPA panels.
 #include "gemm_i8.hpp"
 
 #include <atomic>
@@ -175,6 +175,13 @@ static uint64_t tile256_min_tiles() {
     return (uint64_t)n;
 }
 
+// The few-row kernel above 128 rows, in workgroups of 64 rows x 16 columns,
+// up to this many per CU: dense_i8 512 x 512 x 4096 (256 workgroups; 16
+// 128-tiles) 23.0 -> 11.9 us, 129 x 1000 x 2000 15.5 -> 8.8; at two per CU
+// (512 x 1024 x 4096) the tiles are as fast, above that faster (1000 x 1000 x
+// 1000, 1008 workgroups: 11.7 us on tiles, 15.0 here).
+constexpr uint64_t kSkinnyPerCu = 1;
+
 template <int BL, bool AU8>
 static int launch_gemm(const GemmParams& p, hipStream_t s) {
     if (p.Mout == 0 || p.Nout == 0) return ANE_OK;
@@ -184,7 +191,7 @@ static int launch_gemm(const GemmParams& p, hipStream_t s) {
         const uint64_t tiles256 = (uint64_t)((p.Mout + 255) / 256) * ((p.Nout + 255) / 256);
         const bool e256 = tile256_eligible(p);
         if (e256 && tiles256 >= tile256_min_tiles()) return launch_gemm_tile256(p, s);
-        if (skinny_eligible(p)) return launch_gemm_skinny(p, s);
+        if (skinny_eligible(p, kSkinnyPerCu * tile256_min_tiles())) return launch_gemm_skinny(p, s);
         if (tile128_eligible(p)) {
             // one 128-tile per CU or fewer: the deeper ring; more: two per CU
             const uint64_t tiles128 = (uint64_t)((p.Mout + 127) / 128) * ((p.Nout + 127) / 128);
@@ -192,6 +199,17 @@ static int launch_gemm(const GemmParams& p, hipStream_t s) {
             return launch_gemm_tile128(p, s);
         }
         if (e256) return launch_gemm_tile256(p, s);
+    }
+    if (BL == kBPanel) {
+        // the same choice on panels; k_gemm_i8 is left with operands past the
+        // 32-bit buffer offsets.  dense_i8 before (k_gemm_i8: unpipelined
+        // tiles, B scattered into LDS by dwords) and now: 4096^3 203 -> 72 us
+        // (1.9 POPS), 2048 x 4096 x 4096 103 -> 48, 16 x 4096 x 4096 65 -> 8.0,
+        // 50 x 128 x 784 (uint8 A) 20.8 -> 8.0, 1000^3 28 -> 11.7.
+        const uint64_t tiles256 = (uint64_t)((p.Mout + 255) / 256) * ((p.Nout + 255) / 256);
+        if (tiles256 >= tile256_min_tiles() && panel256_eligible(p)) return launch_gemm_panel256(p, AU8, s);
+        if (panel_skinny_eligible(p, kSkinnyPerCu * tile256_min_tiles())) return launch_gemm_panel_skinny(p, AU8, s);
+        if (panel128_eligible(p)) return launch_gemm_panel128(p, AU8, s);
     }
     dim3 grid((p.Nout + kBN - 1) / kBN, (p.Mout + kBM - 1) / kBM);
     if (grid.y > 65535) return ANE_ERR_INVALID_ARG;

@@ -76,9 +76,22 @@ int launch_gemm_tile128(const GemmParams& p, hipStream_t s, uint32_t ksplit = 1)
 bool tile128d_eligible(const GemmParams& p, bool any_rows = false);
 int launch_gemm_tile128d(const GemmParams& p, hipStream_t s, uint32_t ksplit = 1);
 
-// Few-row kernel (gemm_i8_skinny.hip): Bt layout, signed A, M <= 128, one
-// workgroup per 16 columns.
-bool skinny_eligible(const GemmParams& p);
+// The same loop with B in SMOPA panels (ldb = Kp / 4 groups of 64 bytes per
+// panel) and A int8 or uint8, at 256 x 256 (gemm_i8_panel256.hip) and 128 x
+// 128 tiles (gemm_i8_panel128.hip).  Rows and columns past the operands'
+// ends read as zeros.
+bool panel256_eligible(const GemmParams& p);
+int launch_gemm_panel256(const GemmParams& p, bool a_unsigned, hipStream_t s);
+bool panel128_eligible(const GemmParams& p);
+int launch_gemm_panel128(const GemmParams& p, bool a_unsigned, hipStream_t s);
+
+// Few-row kernel (gemm_i8_skinny.hip): Bt layout, signed A, one workgroup per
+// 16 columns and up to 128 rows, or per 16 columns and 64 rows while that is
+// at most wgs_max workgroups.
+bool skinny_eligible(const GemmParams& p, uint64_t wgs_max);
 int launch_gemm_skinny(const GemmParams& p, hipStream_t s);
+// The same on SMOPA panels, one workgroup per panel, A int8 or uint8.
+bool panel_skinny_eligible(const GemmParams& p, uint64_t wgs_max);
+int launch_gemm_panel_skinny(const GemmParams& p, bool a_unsigned, hipStream_t s);
 
 }  // namespace ane

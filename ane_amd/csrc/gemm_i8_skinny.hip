@@ -34,22 +34,30 @@
 namespace ane {
 namespace {
 
-template <int MB>
+// PANEL: B in the SMOPA panels of dense_i8 / dense_u8s8, workgroup = panel: a
+// lane's 16 bytes of column n0 + l%16 are dword l%16 of four consecutive
+// 64-byte groups.  AU8: uint8 A enters as a - 128 and 128 * (column sum of B)
+// is added back.
+template <int MB, bool PANEL = false, bool AU8 = false>
 __global__ void __launch_bounds__(256) k_gemm_skinny(GemmParams p) {
     __shared__ v4i red[4][MB][64];
+    __shared__ int csum[AU8 ? 4 : 1][16];
     const uint32_t lane = threadIdx.x & 63, c16 = lane & 15, g = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t n0 = blockIdx.x * 16;
     const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.A, (uint32_t)(p.rowsA * p.lda));
-    const __amdgpu_buffer_rsrc_t rb = make_rsrc(p.B, (uint32_t)(p.colsB * p.ldb));
+    const __amdgpu_buffer_rsrc_t rb =
+        make_rsrc(p.B, PANEL ? (uint32_t)((p.colsB + 15) / 16 * p.ldb * 64) : (uint32_t)(p.colsB * p.ldb));
     const uint32_t nsteps = (p.Kp + 127) / 128;  // the last step may be partial: k < Kp decides per chunk
     const uint32_t nj = (nsteps + 3) / 4;  // this wave's steps, rounded up (extra steps read zeros)
     // the rotation of this workgroup's walk (4+ row blocks)
     const uint32_t phase = MB >= 4 ? (blockIdx.x & 3) * (nsteps / 4) : 0;
-    const uint32_t offB = (n0 + c16) * (uint32_t)p.ldb + 32 * g;
+    const uint32_t offB = PANEL ? blockIdx.x * (uint32_t)p.ldb * 64 + 8 * g * 64 + 4 * c16
+                                : (n0 + c16) * (uint32_t)p.ldb + 32 * g;
+    const uint32_t m0 = blockIdx.y * (16 * MB);  // first row of this workgroup
     uint32_t offA[MB];
 #pragma unroll
-    for (int r = 0; r < MB; r++) offA[r] = (16 * r + c16) * (uint32_t)p.lda + 32 * g;
+    for (int r = 0; r < MB; r++) offA[r] = (m0 + 16 * r + c16) * (uint32_t)p.lda + 32 * g;
 
     // step j of this wave: 16-byte chunks h = 0, 1 at k = 128 S + 32 g + 16 h
     auto load = [&](uint32_t j, v4i (&b)[2], v4i (&a)[2][MB]) {
@@ -59,19 +67,35 @@ __global__ void __launch_bounds__(256) k_gemm_skinny(GemmParams p) {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const bool live = in && 128 * S + 32 * g + 16 * h < p.Kp;
-            b[h] = __builtin_bit_cast(
-                v4i, __builtin_amdgcn_raw_buffer_load_b128(rb, live ? offB + 128 * S + 16 * h : 0x80000000u, 0, kCpolNt));
+            if (PANEL) {
+                const uint32_t o = live ? offB + (32 * S + 4 * h) * 64 : 0x80000000u;  // group 32S + 8g + 4h
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    b[h][q] = (int)__builtin_amdgcn_raw_buffer_load_b32(rb, o + 64 * q, 0, kCpolNt);
+            } else {
+                b[h] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                                                   rb, live ? offB + 128 * S + 16 * h : 0x80000000u, 0, kCpolNt));
+            }
 #pragma unroll
             for (int r = 0; r < MB; r++)
                 a[h][r] = __builtin_bit_cast(
                     v4i, __builtin_amdgcn_raw_buffer_load_b128(ra, live ? offA[r] + 128 * S + 16 * h : 0x80000000u, 0, 0));
         }
     };
+    int cs = 0;  // AU8: this lane's share of its column's sum
     auto mma = [&](v4i (&acc)[MB], const v4i (&b)[2], const v4i (&a)[2][MB]) {
+        constexpr int kFlip = AU8 ? (int)0x80808080 : 0;
 #pragma unroll
-        for (int h = 0; h < 2; h++)
+        for (int h = 0; h < 2; h++) {
 #pragma unroll
-            for (int r = 0; r < MB; r++) acc[r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[h][r], b[h], acc[r], 0, 0, 0);
+            for (int r = 0; r < MB; r++)
+                acc[r] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[h][r] ^ v4i{kFlip, kFlip, kFlip, kFlip}, b[h],
+                                                               acc[r], 0, 0, 0);
+            if (AU8) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) cs = __builtin_amdgcn_sdot4(b[h][q], 0x01010101, cs, false);
+            }
+        }
     };
 
     v4i acc[MB];
@@ -88,17 +112,28 @@ __global__ void __launch_bounds__(256) k_gemm_skinny(GemmParams p) {
 
 #pragma unroll
     for (int r = 0; r < MB; r++) red[wave][r][lane] = acc[r];
+    if (AU8) {
+        cs += __shfl_xor(cs, 16, 64);
+        cs += __shfl_xor(cs, 32, 64);
+        if (g == 0) csum[wave][c16] = cs;
+    }
     __syncthreads();
+    const uint32_t add =
+        AU8 ? 128u * (uint32_t)(csum[0][c16] + csum[AU8 ? 1 : 0][c16] + csum[AU8 ? 2 : 0][c16] + csum[AU8 ? 3 : 0][c16])
+            : 0u;
 
     float s = p.s;
     if (p.sdev) s = __fmul_rn(__fmul_rn(p.sdev[0], p.sdev[1]), p.smul);
     const uint32_t j = n0 + c16;
     const float bj = (p.bias && j < p.Nout) ? p.bias[j] : 0.0f;
     for (uint32_t r = wave; r < (uint32_t)MB; r += 4) {
-        const v4i t = red[0][r][lane] + red[1][r][lane] + red[2][r][lane] + red[3][r][lane];
+        v4i t = red[0][r][lane] + red[1][r][lane] + red[2][r][lane] + red[3][r][lane];
+        if (AU8)
+#pragma unroll
+            for (int i = 0; i < 4; i++) t[i] = (int)((uint32_t)t[i] + add);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const uint32_t row = 16 * r + 4 * g + i;
+            const uint32_t row = m0 + 16 * r + 4 * g + i;
             if (row >= p.Mout || j >= p.Nout) continue;
             if (p.Craw) {
                 p.Craw[(uint64_t)row * p.ldc + j] = t[i];
@@ -112,34 +147,55 @@ __global__ void __launch_bounds__(256) k_gemm_skinny(GemmParams p) {
 
 }  // namespace
 
-bool skinny_eligible(const GemmParams& p) {
-    if (p.Mout == 0 || p.Mout > 128 || p.Nout == 0) return false;
+// More than 128 rows: 64-row groups of workgroups while the launch stays
+// within wgs_max workgroups (few 128 x 128 tiles leave most CUs idle).
+static bool rows_ok(const GemmParams& p, uint64_t wgs_max) {
+    return p.Mout <= 128 || (uint64_t)((p.Mout + 63) / 64) * ((p.Nout + 15) / 16) <= wgs_max;
+}
+
+bool skinny_eligible(const GemmParams& p, uint64_t wgs_max) {
+    if (p.Mout == 0 || !rows_ok(p, wgs_max) || p.Nout == 0) return false;
     if (p.Kp == 0 || (p.Kp & 15)) return false;
     if ((p.lda & 15) || (p.ldb & 15)) return false;
     if ((((uintptr_t)p.A) & 15) || (((uintptr_t)p.B) & 15)) return false;
     if (p.rowsA < p.Mout || p.colsB < p.Nout) return false;
     // 32-bit buffer offsets; 0x80000000 marks an empty load: every row a
-    // workgroup may touch (up to 16 past the last column, 128 A rows) and
+    // workgroup may touch (up to 16 past the last column, 128 past the last A row) and
     // every step stay below it
     const uint64_t kspan = ceil_to(p.Kp, 256) + 128;
     if ((uint64_t)ceil_to(p.Nout, 16) * p.ldb + kspan >= (1ull << 31)) return false;
-    if (128ull * p.lda + kspan >= (1ull << 31)) return false;
+    if (ceil_to(p.Mout, 128) * p.lda + kspan >= (1ull << 31)) return false;
     if ((uint64_t)p.rowsA * p.lda >= (1ull << 31) || (uint64_t)p.colsB * p.ldb >= (1ull << 31)) return false;
     return true;
 }
 
-int launch_gemm_skinny(const GemmParams& p, hipStream_t s) {
-    const uint32_t mb = (p.Mout + 15) / 16;
-    const dim3 grid((p.Nout + 15) / 16);
-    switch (mb) {
-        case 1: hipLaunchKernelGGL(k_gemm_skinny<1>, grid, dim3(256), 0, s, p); break;
-        case 2: hipLaunchKernelGGL(k_gemm_skinny<2>, grid, dim3(256), 0, s, p); break;
-        case 3:
-        case 4: hipLaunchKernelGGL(k_gemm_skinny<4>, grid, dim3(256), 0, s, p); break;
-        default: hipLaunchKernelGGL(k_gemm_skinny<8>, grid, dim3(256), 0, s, p); break;
-    }
+template <bool PANEL, bool AU8>
+static int launch_skinny(const GemmParams& p, hipStream_t s) {
+    const uint32_t mb = p.Mout > 128 ? 4 : (p.Mout + 15) / 16;
+    const dim3 grid((p.Nout + 15) / 16, p.Mout > 128 ? (p.Mout + 63) / 64 : 1);
+    const auto fn = mb == 1   ? k_gemm_skinny<1, PANEL, AU8>
+                    : mb == 2 ? k_gemm_skinny<2, PANEL, AU8>
+                    : mb <= 4 ? k_gemm_skinny<4, PANEL, AU8>
+                              : k_gemm_skinny<8, PANEL, AU8>;
+    hipLaunchKernelGGL(fn, grid, dim3(256), 0, s, p);
     ANE_HIP_CHECK_LAUNCH();
     return ANE_OK;
+}
+
+int launch_gemm_skinny(const GemmParams& p, hipStream_t s) { return launch_skinny<false, false>(p, s); }
+
+bool panel_skinny_eligible(const GemmParams& p, uint64_t wgs_max) {
+    if (p.Mout == 0 || !rows_ok(p, wgs_max) || p.Nout == 0 || p.Kp == 0 || (p.Kp & 63) || p.ldb * 4 != p.Kp) return false;
+    if ((p.lda & 15) || (((uintptr_t)p.A) & 15) || (((uintptr_t)p.B) & 15)) return false;
+    if (p.rowsA < p.Mout || p.colsB < p.Nout) return false;
+    // 32-bit buffer offsets, as above: 16 bytes of a panel per byte of K
+    const uint64_t kspan = ceil_to(p.Kp, 256) + 128;
+    return ceil_to(p.colsB, 16) * p.Kp + 16 * kspan < (1ull << 31) && ceil_to(p.Mout, 128) * p.lda + kspan < (1ull << 31) &&
+           (uint64_t)p.rowsA * p.lda < (1ull << 31);
+}
+
+int launch_gemm_panel_skinny(const GemmParams& p, bool a_unsigned, hipStream_t s) {
+    return a_unsigned ? launch_skinny<true, true>(p, s) : launch_skinny<true, false>(p, s);
 }
 
 }  // namespace ane

@@ -78,6 +78,11 @@ namespace {
 #ifndef ANE_TILE_STAGES
 #define ANE_TILE_STAGES 2
 #endif
+// ANE_TILE_PANEL: B in the SMOPA panel format of dense_i8 / dense_u8s8
+// (gemm_i8_panel256.hip, gemm_i8_panel128.hip) instead of rows of Bt.
+#ifndef ANE_TILE_PANEL
+#define ANE_TILE_PANEL 0
+#endif
 
 constexpr int TM = ANE_TILE, TN = ANE_TILE;
 constexpr int TK = 128;                       // bytes of K per slice
@@ -99,9 +104,12 @@ constexpr int kRowsPerDma = 1024 / TK;        // rows covered by one copy wave-i
 constexpr int kRowsPerWave = TM / NW;         // rows of A (and of Bt) each wave copies
 constexpr int kDmaPerWave = kRowsPerWave / kRowsPerDma;
 constexpr int kSteps = TK / 32;
+constexpr bool kPanel = ANE_TILE_PANEL;
+constexpr int kCopies = kPanel ? kDmaPerWave : 2 * kDmaPerWave;  // copies to LDS per wave and slice
 static_assert(NW == 4 || NW == 8 || NW == 16, "4, 8 or 16 waves");
 static_assert(STAGES >= 2 && (STAGES - 2) * 2 * kDmaPerWave < 64, "ring depth fits the vmcnt field");
 static_assert(kLdsBytes <= 160 * 1024, "LDS ring exceeds 160 KB");
+static_assert(!kPanel || (STAGES == 2 && TN * 2 == kThreads), "one panel unit per thread and slice");
 // Epilogue staging: per wave EPR rows x (FN*32) fp32 per pass, rows padded
 // by 32 bytes (4 rows apart = 128 bytes mod 256: the two half-waves of a
 // staging write land in different bank halves).
@@ -166,18 +174,20 @@ __device__ __forceinline__ void load_frag(const int8_t* stage, uint32_t rA, uint
 }
 
 // One slice: the copies of the next slice and the next k-step's fragment
-// reads pinned between the MFMAs.  f0 holds the slice's first fragments on
-// entry.
+// reads pinned between the MFMAs, with extra(ks, g) after MFMA g of k-step
+// ks.  f0 holds the slice's first fragments on entry.  amask: XORed into A
+// (0, or 0x80 per byte for uint8 A, whose bytes then enter as a - 128).
+template <class Extra>
 __device__ __forceinline__ void slice_pinned(v16i (&acc)[FM][FN], Frags& f0, Frags& f1, const int8_t* cur,
                                              uint32_t rA, uint32_t rB, uint32_t chalf, const SliceCopy& c,
                                              const uint32_t (&offA)[kDmaPerWave],
                                              const uint32_t (&offB)[kDmaPerWave],
-                                             const uint32_t (&kofs)[kDmaPerWave]) {
+                                             const uint32_t (&kofs)[kDmaPerWave], int amask, Extra&& extra) {
     constexpr int nM = FM * FN, nD = FM + FN;
-    constexpr int kCopySteps = 2;                       // k-steps that carry the copies
-    constexpr int kPerStep = 2 * kDmaPerWave / kCopySteps;
+    constexpr int kCopySteps = kPanel ? 1 : 2;          // k-steps that carry the copies
+    constexpr int kPerStep = kCopies / kCopySteps;
     constexpr int kStride = nM / kPerStep;              // MFMAs per copy
-    static_assert(kPerStep * kCopySteps == 2 * kDmaPerWave && kStride * kPerStep == nM && kCopySteps <= kSteps,
+    static_assert(kPerStep * kCopySteps == kCopies && kStride * kPerStep == nM && kCopySteps <= kSteps,
                   "copies must spread evenly over the MFMAs");
 #pragma unroll
     for (int ks = 0; ks < kSteps; ks++) {
@@ -186,10 +196,12 @@ __device__ __forceinline__ void slice_pinned(v16i (&acc)[FM][FN], Frags& f0, Fra
 #pragma unroll
         for (int g = 0; g < nM; g++) {
             const int mi = g / FN, ni = g % FN;
-            acc[mi][ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fc.a[mi], fc.b[ni], acc[mi][ni], 0, 0, 0);
+            const v4i a = amask ? fc.a[mi] ^ v4i{amask, amask, amask, amask} : fc.a[mi];
+            acc[mi][ni] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, fc.b[ni], acc[mi][ni], 0, 0, 0);
             if (ks + 1 < kSteps && g < nD) load_frag(cur, rA, rB, 2 * (ks + 1) + chalf, fn, g);
             if (ks < kCopySteps && g % kStride == kStride - 1)
                 issue_one(c, offA, offB, kofs, ks * kPerStep + g / kStride);
+            extra(ks, g);
             __builtin_amdgcn_sched_barrier(0);
         }
         // fewer MFMAs than fragments per k-step (1 x 2 blocks per wave): the
@@ -200,6 +212,41 @@ __device__ __forceinline__ void slice_pinned(v16i (&acc)[FM][FN], Frags& f0, Fra
         __builtin_amdgcn_sched_barrier(0);
     }
 }
+
+#if ANE_TILE_PANEL
+// B panels -> the LDS rows the fragments read.  A slice of one panel is 32
+// groups of 64 bytes; a thread takes the unit (panel, 4 groups, 4 columns):
+// one 16-byte load per group (4 columns x 4 k), and then, with no
+// arithmetic, dword c of the four loads is the 16-byte chunk of column c.
+// The loads of slice kt+2 are in flight while slice kt is multiplied and
+// slice kt+1's chunks are written.
+struct PanelB {
+    __amdgpu_buffer_rsrc_t rb;
+    uint32_t off, lds[4], k;  // byte of group 0 of the unit; LDS offsets of its four columns; its k in a slice
+    v4u v[4];
+    __device__ __forceinline__ void setup(const GemmParams& p, uint32_t tid, uint32_t col0, __amdgpu_buffer_rsrc_t r) {
+        const uint32_t cq = tid & 3, gq = (tid >> 2) & 7, panel = tid >> 5;
+        rb = r;
+        k = gq * 16;
+        off = (((col0 >> 4) + panel) * (uint32_t)p.ldb + gq * 4) * 64 + cq * 16;
+#pragma unroll
+        for (uint32_t c = 0; c < 4; c++) lds[c] = kStageA + swz(panel * 16 + cq * 4 + c, gq);
+    }
+    // group i of slice at byte k0 of K, zeros past kmax bytes of the slice
+    __device__ __forceinline__ void load(uint32_t i, uint32_t k0, uint32_t kmax) {
+        v[i] = __builtin_amdgcn_raw_buffer_load_b128(rb, k < kmax ? off + k0 * 16 + i * 64 : 0x80000000u, 0, 0);
+    }
+    __device__ __forceinline__ void store(uint32_t c, int8_t* stage) {
+        const v4u w = {v[0][c], v[1][c], v[2][c], v[3][c]};
+        asm volatile("ds_write_b128 %0, %1" ::"v"(lds_offset(stage) + lds[c]), "v"(w) : "memory");
+    }
+    __device__ __forceinline__ int sum(uint32_t c, int s) const {  // s + the column's signed bytes
+#pragma unroll
+        for (int i = 0; i < 4; i++) s = __builtin_amdgcn_sdot4((int)v[i][c], 0x01010101, s, false);
+        return s;
+    }
+};
+#endif
 
 // A whole 16-byte store of C with the sc1 bit (agent scope): the line is
 // written through the XCD's L2 instead of being left dirty there for the
@@ -216,6 +263,11 @@ __device__ __forceinline__ void store16_sc1(uint32_t* dst, v4i v) {
     asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(dst), "v"(v) : "memory");
 }
 
+#if ANE_TILE_PANEL
+template <bool AU8>
+#else
+constexpr bool AU8 = false;
+#endif
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWavesPerEu, kWavesPerEu)))
 ANE_TILE_KERNEL(GemmParams p, uint32_t tiles_m, uint32_t tiles_n) {
     __shared__ __attribute__((aligned(1024))) int8_t smem[kLdsBytes];
@@ -239,7 +291,9 @@ ANE_TILE_KERNEL(GemmParams p, uint32_t tiles_m, uint32_t tiles_n) {
     const uint32_t col0 = (in / gm) * TN;
 
     const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.A, (uint32_t)(p.rowsA * p.lda));
-    const __amdgpu_buffer_rsrc_t rb = make_rsrc(p.B, (uint32_t)(p.colsB * p.ldb));
+    // panels: ldb groups of 64 bytes per 16 columns
+    const __amdgpu_buffer_rsrc_t rb =
+        make_rsrc(p.B, kPanel ? (uint32_t)((p.colsB + 15) / 16 * p.ldb * 64) : (uint32_t)(p.colsB * p.ldb));
     uint32_t offA[kDmaPerWave], offB[kDmaPerWave], kofs[kDmaPerWave];
     {
         // lane l fills slot l % kChunks of row wave*kRowsPerWave + i*kRowsPerDma + l/kChunks
@@ -250,7 +304,7 @@ ANE_TILE_KERNEL(GemmParams p, uint32_t tiles_m, uint32_t tiles_n) {
             const uint32_t chunk = (lane % kChunks) ^ swz_g(row);
             kofs[i] = chunk * 16;
             offA[i] = (row0 + row) * (uint32_t)p.lda + kofs[i];
-            offB[i] = (col0 + row) * (uint32_t)p.ldb + kofs[i];
+            offB[i] = kPanel ? 0u : (col0 + row) * (uint32_t)p.ldb + kofs[i];
         }
     }
 
@@ -289,13 +343,32 @@ ANE_TILE_KERNEL(GemmParams p, uint32_t tiles_m, uint32_t tiles_n) {
     for (int j = 0; j < STAGES - 1; j++) {
         const SliceCopy c{ra, rb, smem + j * kStage, wave, (kt0 + j) * TK, kmax(kt0 + j)};
 #pragma unroll
-        for (int d = 0; d < 2 * kDmaPerWave; d++) issue_one(c, offA, offB, kofs, d);
+        for (int d = 0; d < kCopies; d++) issue_one(c, offA, offB, kofs, d);
     }
+#if ANE_TILE_PANEL
+    PanelB pb;
+    pb.setup(p, tid, col0, rb);
+    int csum[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) pb.load(i, 0, kmax(0));
+#pragma unroll
+    for (uint32_t c = 0; c < 4; c++) {
+        pb.store(c, smem);
+        if (AU8) csum[c] = pb.sum(c, csum[c]);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) pb.load(i, TK, kmax(1));
+#endif
     uint32_t st = 0;  // stage of slice kt
     for (uint32_t kt = kt0; kt < kt1; kt++) {
         // this wave's copies of slice kt landed (those of the STAGES-2
         // slices after it may still be in flight; copies complete in order)
-        wait_vmcnt<(STAGES - 2) * 2 * kDmaPerWave>();
+        if (kPanel) {
+            wait_vmcnt<4>();  // all but the four loads of slice kt+1's panels
+            wait_lgkmcnt0();  // this wave's chunks of slice kt are written
+        } else {
+            wait_vmcnt<(STAGES - 2) * 2 * kDmaPerWave>();
+        }
         lds_barrier();    // everyone's did; everyone finished slice kt-1
         const int8_t* cur = smem + st * kStage;
         const uint32_t sn = st == 0 ? STAGES - 1 : st - 1;  // slice kt-1's stage takes slice kt+STAGES-1
@@ -303,11 +376,45 @@ ANE_TILE_KERNEL(GemmParams p, uint32_t tiles_m, uint32_t tiles_n) {
         st = st + 1 == STAGES ? 0 : st + 1;
         load_frags(cur, rA, rB, chalf, f0);
         __builtin_amdgcn_sched_barrier(0);
-        slice_pinned(acc, f0, f1, cur, rA, rB, chalf, c, offA, offB, kofs);
+#if ANE_TILE_PANEL
+        int8_t* next = smem + sn * kStage;
+        const uint32_t k2 = (kt + 2) * TK, kmax2 = kmax(kt + 2);
+        slice_pinned(acc, f0, f1, cur, rA, rB, chalf, c, offA, offB, kofs, AU8 ? (int)0x80808080 : 0,
+                     [&](int ks, int g) {
+                         constexpr int q = FM * FN / 4;  // one of four per q MFMAs
+                         if (g % q != q - 1) return;
+                         if (ks == 1) {
+                             pb.store(g / q, next);
+                             if (AU8) csum[g / q] = pb.sum(g / q, csum[g / q]);
+                         }
+                         if (ks == 2) pb.load(g / q, k2, kmax2);
+                     });
+#else
+        slice_pinned(acc, f0, f1, cur, rA, rB, chalf, c, offA, offB, kofs, 0, [](int, int) {});
+#endif
     }
     wait_vmcnt<0>();
     __syncthreads();  // all fragment reads done: the ring becomes epilogue staging
 
+#if ANE_TILE_PANEL
+    // uint8 A: the accumulators hold sum (a - 128) b; add 128 * column sum of b
+    int csj[FN];
+    if (AU8) {
+        int* sums = reinterpret_cast<int*>(smem);  // one per tile column
+#pragma unroll
+        for (uint32_t c = 0; c < 4; c++) {  // fold the eight k-units of the column: lane bits 2..4
+            int v = csum[c];
+            v += __shfl_xor(v, 4, 64);
+            v += __shfl_xor(v, 8, 64);
+            v += __shfl_xor(v, 16, 64);
+            if ((tid & 28) == 0) sums[(tid >> 5) * 16 + (tid & 3) * 4 + c] = v;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int ni = 0; ni < FN; ni++) csj[ni] = sums[wc0 + ni * 32 + (lane & 31)];
+        __syncthreads();
+    }
+#endif
     float bj[FN];
 #pragma unroll
     for (int ni = 0; ni < FN; ni++) {
@@ -331,10 +438,14 @@ ANE_TILE_KERNEL(GemmParams p, uint32_t tiles_m, uint32_t tiles_n) {
                     const uint32_t lr = 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3) - h * EPR;
                     const uint32_t lc = ni * 32 + (lane & 31);
                     uint32_t bitsv;
+                    int32_t av = acc[mi][ni][r];
+#if ANE_TILE_PANEL
+                    if (AU8) av = (int32_t)((uint32_t)av + 128u * (uint32_t)csj[ni]);
+#endif
                     if (craw) {
-                        bitsv = (uint32_t)acc[mi][ni][r];
+                        bitsv = (uint32_t)av;
                     } else {
-                        const float f = __fadd_rn(__fmul_rn((float)acc[mi][ni][r], s), bj[ni]);
+                        const float f = __fadd_rn(__fmul_rn((float)av, s), bj[ni]);
                         bitsv = __float_as_uint(fmax_a(f, p.lo));
                     }
                     *reinterpret_cast<uint32_t*>(epi + lr * kEpiRowBytes + lc * 4) = bitsv;
@@ -370,6 +481,26 @@ ANE_TILE_KERNEL(GemmParams p, uint32_t tiles_m, uint32_t tiles_n) {
 
 }  // namespace
 
+#if ANE_TILE_PANEL
+bool ANE_TILE_ELIGIBLE(const GemmParams& p) {
+    if (p.Mout == 0 || p.Nout == 0 || p.Kp == 0 || (p.Kp % 64) || p.ldb * 4 != p.Kp) return false;
+    if ((p.lda & 15) || (((uintptr_t)p.A) & 15) || (((uintptr_t)p.B) & 15)) return false;
+    if (p.rowsA < p.Mout || p.colsB < p.Nout) return false;
+    // 32-bit buffer offsets, 0x80000000 marks an empty load
+    const uint64_t rows_a = ceil_to(p.Mout, TM) + TM, cols_b = ceil_to(p.Nout, TN) + TN;
+    return rows_a * p.lda + p.Kp < (1ull << 31) && cols_b * p.Kp + 32ull * TK * 16 < (1ull << 31);
+}
+
+int ANE_TILE_LAUNCH(const GemmParams& p, bool a_unsigned, hipStream_t s) {
+    const uint32_t tiles_m = (p.Mout + TM - 1) / TM, tiles_n = (p.Nout + TN - 1) / TN;
+    const uint64_t total = (uint64_t)tiles_m * tiles_n;
+    if (total > 0x7fffffffull) return ANE_ERR_INVALID_ARG;
+    const auto fn = a_unsigned ? ANE_TILE_KERNEL<true> : ANE_TILE_KERNEL<false>;
+    hipLaunchKernelGGL(fn, dim3((uint32_t)total), dim3(kThreads), 0, s, p, tiles_m, tiles_n);
+    ANE_HIP_CHECK_LAUNCH();
+    return ANE_OK;
+}
+#else
 bool ANE_TILE_ELIGIBLE(const GemmParams& p, bool any_rows) {
     if ((!any_rows && p.Mout < TM) || p.Nout < TN) return false;
     if (p.Kp == 0 || (p.Kp % 64) != 0) return false;
@@ -395,5 +526,6 @@ int ANE_TILE_LAUNCH(const GemmParams& p, hipStream_t s, uint32_t ksplit) {
     ANE_HIP_CHECK_LAUNCH();
     return ANE_OK;
 }
+#endif
 
 }  // namespace ane
