@@ -71,6 +71,13 @@ __device__ float frsqrte_a(float x) {
     return f_of(((uint32_t)(rexp & 0xff) << 23) | ((est & 0xff) << 15));
 }
 
+// floor(2^19 / d) for odd d in [513, 1023]: the quotient is at least 2^-10
+// away from any integer and below 2^10, and the product of 2^19 and the 1-ulp
+// reciprocal is off by less than 2^-12.
+__device__ __forceinline__ uint32_t recip_quotient(uint32_t d) {
+    return (uint32_t)(524288.0f * __builtin_amdgcn_rcpf((float)d));
+}
+
 __device__ __forceinline__ float frecpe_a(float x) {
     const uint32_t u = __float_as_uint(x), sign = u >> 31, ex = (u >> 23) & 0xff, fr = u & 0x7fffff;
     if (ex == 0xff && fr) return f_of(u | 0x00400000u);
@@ -88,7 +95,7 @@ __device__ __forceinline__ float frecpe_a(float x) {
     }
     const uint32_t scaled = 256u + (uint32_t)(f52 >> 44);
     int rexp = 253 - e;
-    const uint32_t est = ((1u << 19) / (scaled * 2 + 1) + 1) / 2;
+    const uint32_t est = (recip_quotient(scaled * 2 + 1) + 1) / 2;
     uint64_t frac = (uint64_t)(est & 0xff) << 44;
     if (rexp == 0) {
         frac = (1ull << 51) | (frac >> 1);
@@ -109,12 +116,12 @@ __device__ __forceinline__ float frecps_a(float a, float b) {
     return inf_times_zero(a, b) ? 2.0f : __builtin_fmaf(-a, b, 2.0f);
 }
 
-// fcvtzs to int32: truncation, saturating, NaN -> 0.
+// fcvtzs to int32: truncation, saturating, NaN -> 0, which is what
+// v_cvt_i32_f32 does (a C cast is undefined out of range).
 __device__ __forceinline__ int32_t cvtzs_a(float x) {
-    if (x != x) return 0;
-    if (x >= 2147483648.0f) return 0x7fffffff;
-    if (x <= -2147483648.0f) return (int32_t)0x80000000u;
-    return (int32_t)x;
+    int32_t r;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
 }
 
 // The handlers' exp approximation (:6627-6665, :6965-6989): 2^n injected as
@@ -136,12 +143,25 @@ __device__ __forceinline__ float exp_poly_a(float x, bool clamp) {
     return __fmul_rn(p, f_of(((uint32_t)ni + 127u) << 23));
 }
 
+// For |x| < 80 (e and d finite, d in [1, 2^116)) the estimate needs no special
+// cases and no Newton step meets inf * 0: the same operations on the same
+// values without the tests.
 __device__ __forceinline__ float silu_a(float x) {
     const float e = exp_poly_a(-x, true);
     const float d = __fadd_rn(e, 1.0f);
-    float r = frecpe_a(d);
-    r = __fmul_rn(r, frecps_a(d, r));
-    r = __fmul_rn(r, frecps_a(d, r));
+    float r;
+    if (__builtin_expect(__builtin_fabsf(x) < 80.0f, 1)) {
+        const uint32_t u = __float_as_uint(d);
+        const uint32_t div = ((u >> 14) & 0x1fe) + 513u;  // 2 (256 + the top 8 mantissa bits) + 1
+        const uint32_t est = (recip_quotient(div) + 1) / 2;
+        r = f_of((0x7e800000u - (u & 0x7f800000u)) | ((est & 0xff) << 15));  // exponent 253 - e
+        r = __fmul_rn(r, __builtin_fmaf(-d, r, 2.0f));
+        r = __fmul_rn(r, __builtin_fmaf(-d, r, 2.0f));
+    } else {
+        r = frecpe_a(d);
+        r = __fmul_rn(r, frecps_a(d, r));
+        r = __fmul_rn(r, frecps_a(d, r));
+    }
     return __fmul_rn(x, r);
 }
 
@@ -166,13 +186,17 @@ __device__ float rope_ratio_a(uint32_t dim, float theta) {
 
 // The rotation of pair p (:6827-6905): power = ratio^(p mod 16) by
 // sequential products, times ratio^16 once per earlier 16-pair chunk.
-__device__ __forceinline__ float2 rope_pair_a(float a, float b, uint32_t p, float ratio, float posf) {
+__device__ __forceinline__ float rope_power_a(uint32_t p, float ratio) {
     float power = 1.0f, r16 = 1.0f;
     for (uint32_t k = 0; k < 16; k++) {
         if (k == (p & 15)) power = r16;
         r16 = __fmul_rn(r16, ratio);
     }
     for (uint32_t c = 0; c < (p >> 4); c++) power = __fmul_rn(power, r16);
+    return power;
+}
+
+__device__ __forceinline__ float2 rope_rotate_a(float a, float b, float power, float posf) {
     const float freq = __fdiv_rn(posf, power);
     const float nq = __builtin_rintf(__fmul_rn(freq, f_of(0x3EA2F983u)));
     const uint32_t odd = ((uint32_t)cvtzs_a(nq) & 1u) << 31;
@@ -196,13 +220,12 @@ __device__ __forceinline__ float2 rope_pair_a(float a, float b, uint32_t p, floa
     return make_float2(oe, oo);
 }
 
-// NaN-propagating FMAX (AArch64, not FMAXNM): max(+0, -0) = +0.
-__device__ __forceinline__ float fmax_nan(float a, float b) {
-    if (a != a) return a;
-    if (b != b) return b;
-    if (a == b) return __float_as_uint(a) >> 31 ? b : a;
-    return a > b ? a : b;
+__device__ __forceinline__ float2 rope_pair_a(float a, float b, uint32_t p, float ratio, float posf) {
+    return rope_rotate_a(a, b, rope_power_a(p, ratio), posf);
 }
+
+// NaN-propagating FMAX (AArch64, not FMAXNM): max(+0, -0) = +0.
+__device__ __forceinline__ float fmax_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 
 constexpr uint32_t kStageFloats = 8192;  // rows up to this long are held in registers and LDS
 
@@ -379,9 +402,18 @@ k_add_rms_norm_ref(uint32_t dim, float eps, float* x, const float* __restrict__ 
     rms_norm_row<true, true>(dim, eps, x, w, xn, y, x);
 }
 
-__global__ void __launch_bounds__(256) k_silu_ref(uint64_t n, const float* __restrict__ in, float* __restrict__ out) {
-    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) out[i] = silu_a(in[i]);
+// Four values per thread (VEC: in and out 16-byte aligned).  VALU-bound at
+// about 35 instructions a value: 4.2 M values 11.2 -> 7.0 us (one value per
+// thread and an integer division in the estimate before).
+template <bool VEC>
+__global__ void __launch_bounds__(256) k_silu_ref(uint64_t n, const float* in, float* out) {
+    const uint64_t i = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (VEC && i + 4 <= n) {
+        const float4 v = *reinterpret_cast<const float4*>(in + i);
+        *reinterpret_cast<float4*>(out + i) = make_float4(silu_a(v.x), silu_a(v.y), silu_a(v.z), silu_a(v.w));
+        return;
+    }
+    for (uint64_t k = i; k < i + 4 && k < n; k++) out[k] = silu_a(in[k]);
 }
 
 // 0x55 over `rows` rows of dim floats (row stride `stride` floats), one
@@ -474,6 +506,101 @@ __global__ void __launch_bounds__(256) k_softmax_ref(uint32_t dim, const float* 
     softmax_row<false>(dim, in + blockIdx.x * stride, out + blockIdx.x * stride, 1.0f, nullptr);
 }
 
+// Softmax of many short rows (dim <= 16 * NR): 16 lanes per row, lane l
+// holding the row's elements l, l + 16, ... -- chain l of the handler -- in
+// registers, so the maximum and the FADDV are DPP steps within the 16 lanes
+// and nothing goes through LDS.  The row kernel above gives such rows a
+// workgroup each, whose one summing wave leaves three idle: 8192 rows of 512
+// with a mask 59 -> 12.5 us (34.6 MB moved; 6.7 us at the rate of a copy).  The same arithmetic as softmax_row<NODE>.
+template <int NR, bool NODE>
+__global__ void __launch_bounds__(256)
+k_softmax_short(uint32_t dim, uint64_t rows, float scale, const uint8_t* in, NodeRows src, const uint8_t* mask,
+                NodeRows msk, uint8_t* out, NodeRows dst) {
+    static_assert(NR % 8 == 0, "groups of 8");
+    const uint32_t l = threadIdx.x & 15;
+    uint64_t r = (uint64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+    const bool live = r < rows;
+    if (!live) r = rows - 1;  // every lane of a DPP row stays active
+    const RowIdx i = row_index(dst, r);
+    const float* x = reinterpret_cast<const float*>(in + row_offset(src, i));
+    const float* mrow = NODE && mask ? reinterpret_cast<const float*>(mask + row_offset(msk, i)) : nullptr;
+    float* o = reinterpret_cast<float*>(out + row_offset(dst, i));
+    float v[NR];
+    float m = -__builtin_inff();
+#pragma unroll
+    for (uint32_t g = 0; g < NR / 8; g++) {
+        if (g * 128 >= dim) break;
+#pragma unroll
+        for (uint32_t k = g * 8; k < g * 8 + 8; k++) v[k] = x[l + 16 * k < dim ? l + 16 * k : dim - 1];
+        if (NODE) {
+            float w[8];
+#pragma unroll
+            for (uint32_t k = 0; k < 8; k++) {
+                const uint32_t e = l + 16 * (g * 8 + k);
+                w[k] = mrow ? mrow[e < dim ? e : dim - 1] : 0.0f;
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < 8; k++) {
+                v[g * 8 + k] = __fmul_rn(v[g * 8 + k], scale);
+                if (mrow) v[g * 8 + k] = __fadd_rn(v[g * 8 + k], w[k]);
+            }
+        }
+    }
+#pragma unroll
+    for (uint32_t g = 0; g < NR / 8; g++) {
+        if (g * 128 >= dim) break;
+#pragma unroll
+        for (uint32_t k = g * 8; k < g * 8 + 8; k++)
+            if (l + 16 * k < dim) m = fmax_nan(m, v[k]);
+    }
+    m = fmax_nan(m, dpp_f32<kDppQuadXor1>(m));
+    m = fmax_nan(m, dpp_f32<kDppQuadXor2>(m));
+    m = fmax_nan(m, dpp_f32<kDppHalfMirror>(m));
+    m = fmax_nan(m, dpp_f32<kDppRowMirror>(m));
+    float acc = 0.0f;
+#pragma unroll
+    for (uint32_t g = 0; g < NR / 8; g++) {
+        if (g * 128 >= dim) break;
+#pragma unroll
+        for (uint32_t k = g * 8; k < g * 8 + 8; k++) {
+            const float d = __fsub_rn(v[k], m);
+            v[k] = NODE && d == -__builtin_inff() ? 0.0f : exp_poly_a(d, true);
+        }
+#pragma unroll
+        for (uint32_t k = g * 8; k < g * 8 + 8; k++)
+            if (l + 16 * k < dim) acc = __fadd_rn(acc, v[k]);
+    }
+    const float inv = __fdiv_rn(1.0f, faddv16(acc));
+    if (!live) return;
+#pragma unroll
+    for (uint32_t g = 0; g < NR / 8; g++) {
+        if (g * 128 >= dim) break;
+#pragma unroll
+        for (uint32_t k = g * 8; k < g * 8 + 8; k++)
+            if (l + 16 * k < dim) o[l + 16 * k] = __fmul_rn(v[k], inv);
+    }
+}
+
+// Short rows from one wave (four rows) per CU up; fewer rows keep a workgroup
+// each.  False: not this kernel's shape.
+template <bool NODE>
+bool softmax_short_launch(uint32_t dim, uint64_t rows, float scale, const uint8_t* in, const NodeRows& src,
+                          const uint8_t* mask, const NodeRows& msk, uint8_t* out, const NodeRows& dst,
+                          hipStream_t s) {
+    int dev = 0, cus = 0;
+    if (dim > 1024 || rows < 4 || hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        rows < 4ull * (uint64_t)cus)
+        return false;
+    const auto fn = dim <= 128   ? k_softmax_short<8, NODE>
+                    : dim <= 256 ? k_softmax_short<16, NODE>
+                    : dim <= 512 ? k_softmax_short<32, NODE>
+                                 : k_softmax_short<64, NODE>;
+    hipLaunchKernelGGL(fn, dim3((uint32_t)((rows + 15) / 16)), dim3(256), 0, s, dim, rows, scale, in, src, mask, msk,
+                       out, dst);
+    return true;
+}
+
 // ------------------------------------------------------ ggml node forms
 // One workgroup per row of the node (ggml_rows.hpp); the rows' operands
 // may sit anywhere their strides put them.
@@ -493,20 +620,22 @@ k_softmax_node(uint32_t dim, float scale, const uint8_t* in, NodeRows src, const
                       mask ? reinterpret_cast<const float*>(mask + row_offset(msk, i)) : nullptr);
 }
 
-// One thread per pair, grid-stride over rows * dim/2 pairs.  Both values of
-// a pair are read before either is written, so out may alias in.
+// A thread takes one pair of the rows row0, row0 + step, ...: the pair's
+// power of the ratio is computed once.  Both values of a pair are read before
+// either is written, so out may alias in.
 __global__ void __launch_bounds__(256)
-k_rope_node(uint32_t dim, uint64_t total, float theta, const int32_t* __restrict__ pos, const uint8_t* in,
-            NodeRows src, uint8_t* out, NodeRows dst) {
+k_rope_node(uint32_t dim, uint64_t rows, uint64_t step, float theta, const int32_t* __restrict__ pos,
+            const uint8_t* in, NodeRows src, uint8_t* out, NodeRows dst) {
     const uint32_t pairs = dim / 2;
-    const float ratio = rope_ratio_a(dim, theta);
-    for (uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (uint64_t)gridDim.x * 256) {
-        const uint64_t row = t / pairs;
-        const uint32_t p = (uint32_t)(t - row * pairs);
+    const uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x, row0 = row_div(t, pairs);
+    if (row0 >= step) return;
+    const uint32_t p = (uint32_t)(t - row0 * pairs);
+    const float power = rope_power_a(p, rope_ratio_a(dim, theta));
+    for (uint64_t row = row0; row < rows; row += step) {
         const RowIdx i = row_index(dst, row);
         const float* x = reinterpret_cast<const float*>(in + row_offset(src, i));
         float* o = reinterpret_cast<float*>(out + row_offset(dst, i));
-        const float2 v = rope_pair_a(x[2 * p], x[2 * p + 1], p, ratio, (float)pos[i.i2]);
+        const float2 v = rope_rotate_a(x[2 * p], x[2 * p + 1], power, (float)pos[i.i2]);
         o[2 * p] = v.x;
         o[2 * p + 1] = v.y;
     }
@@ -802,6 +931,10 @@ int softmax_node_launch(uint32_t dim, uint64_t rows, float scale, const uint8_t*
                         const uint8_t* mask, const NodeRows& msk, uint8_t* out, const NodeRows& dst, hipStream_t s) {
     if (rows == 0 || dim == 0) return ANE_OK;
     if (rows > 0x7fffffffu) return ANE_ERR_INVALID_ARG;
+    if (softmax_short_launch<true>(dim, rows, scale, in, src, mask, msk, out, dst, s)) {
+        ANE_HIP_CHECK_LAUNCH();
+        return ANE_OK;
+    }
     hipLaunchKernelGGL(k_softmax_node, dim3((uint32_t)rows), dim3(256), 0, s, dim, scale, in, src, mask, msk, out,
                        dst);
     ANE_HIP_CHECK_LAUNCH();
@@ -810,12 +943,16 @@ int softmax_node_launch(uint32_t dim, uint64_t rows, float scale, const uint8_t*
 
 int rope_node_launch(uint32_t dim, uint64_t rows, float theta, const int32_t* pos, const uint8_t* in,
                      const NodeRows& src, uint8_t* out, const NodeRows& dst, hipStream_t s) {
-    const uint64_t total = rows * (dim / 2);
-    if (total == 0) return ANE_OK;
-    uint64_t blocks = (total + 255) / 256;
-    if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(k_rope_node, dim3((uint32_t)blocks), dim3(256), 0, s, dim, total, theta, pos, in, src, out,
-                       dst);
+    if (rows == 0 || dim < 2) return ANE_OK;
+    // 4096 rows per sweep, more where that would be over eight sweeps; at
+    // most 2^24 workgroups
+    const uint32_t pairs = dim / 2;
+    uint64_t step = rows / 8 > 4096 ? rows / 8 : 4096;
+    if (step > rows) step = rows;
+    const uint64_t cap = (1ull << 32) / pairs;
+    if (step > cap) step = cap ? cap : 1;
+    hipLaunchKernelGGL(k_rope_node, dim3((uint32_t)((step * pairs + 255) / 256)), dim3(256), 0, s, dim, rows, step,
+                       theta, pos, in, src, out, dst);
     ANE_HIP_CHECK_LAUNCH();
     return ANE_OK;
 }
@@ -840,9 +977,9 @@ extern "C" int ane_hip_rms_norm_fp32(uint32_t rows, uint32_t dim, float eps, con
 extern "C" int ane_hip_silu_fp32(uint64_t count, const float* in, float* out, void* stream) {
     if (count == 0) return ANE_OK;
     if (!in || !out) return ANE_ERR_BAD_POINTER;
-    const uint64_t blocks = (count + 255) / 256;
-    if (blocks > 0x7fffffffull) return ANE_ERR_INVALID_ARG;
-    hipLaunchKernelGGL(k_silu_ref, dim3((uint32_t)blocks), dim3(256), 0, (hipStream_t)stream, count, in, out);
+    if ((count + 255) / 256 > 0x7fffffffull) return ANE_ERR_INVALID_ARG;
+    const auto fn = ((((uintptr_t)in) | ((uintptr_t)out)) & 15) == 0 ? k_silu_ref<true> : k_silu_ref<false>;
+    hipLaunchKernelGGL(fn, dim3((uint32_t)((count + 1023) / 1024)), dim3(256), 0, (hipStream_t)stream, count, in, out);
     ANE_HIP_CHECK_LAUNCH();
     return ANE_OK;
 }

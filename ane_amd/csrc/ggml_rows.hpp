@@ -24,13 +24,23 @@ struct RowIdx {
     uint64_t i1, i2, i3;
 };
 
+// a / b, in 32 bits where both fit (the 64-bit division is a subroutine of
+// over a hundred instructions, several of them per row).
+__host__ __device__ inline uint64_t row_div(uint64_t a, uint64_t b) {
+    return ((a | b) >> 32) ? a / b : (uint64_t)((uint32_t)a / (uint32_t)b);
+}
+
 __host__ __device__ inline RowIdx row_index(const NodeRows& d, uint64_t r) {
-    const uint64_t q = r / d.ne1;
-    return RowIdx{r - q * d.ne1, q % d.ne2, q / d.ne2};
+    const uint64_t q = row_div(r, d.ne1), i3 = row_div(q, d.ne2);
+    return RowIdx{r - q * d.ne1, q - i3 * d.ne2, i3};
+}
+
+__host__ __device__ inline uint64_t row_repeat(uint64_t i, uint64_t ne) {
+    return i < ne ? i : i - row_div(i, ne) * ne;
 }
 
 __host__ __device__ inline uint64_t row_offset(const NodeRows& m, const RowIdx& i) {
-    return (i.i1 % m.ne1) * m.nb1 + (i.i2 % m.ne2) * m.nb2 + (i.i3 % m.ne3) * m.nb3;
+    return row_repeat(i.i1, m.ne1) * m.nb1 + row_repeat(i.i2, m.ne2) * m.nb2 + row_repeat(i.i3, m.ne3) * m.nb3;
 }
 
 // Row kernels in the reference handlers' arithmetic (decode_ref.hip), one
