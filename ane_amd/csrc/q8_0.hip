@@ -16,12 +16,15 @@
 //    aligned), the matrix is under 2 GB and the activations fit in LDS;
 //  * the MFMA kernels (k_q8_0_mma, k_q8_0_mmt), G mode for 5+ tokens when
 //    nb % 16 == 0;
+//  * the prompt kernel (q8_0_prompt.hip), G mode for many tokens, and for 5+
+//    tokens on rows the kernels above do not take;
 //  * general kernels (k_q8_0_gemv_r, k_q8_0_quantize_x + k_q8_0_mul_mat_g)
 //    for everything else.
 #include "../../include/ane_decode.h"
 #include "common.hpp"
 #include "qformats.hpp"
 #include "q8_0_mmv.hpp"
+#include "q8_0_prompt.hpp"
 
 #include <atomic>
 #include <map>
@@ -91,9 +94,8 @@ k_q8_act_quantize(uint32_t nblocks, uint32_t nb, uint32_t K, const float* __rest
     const uint32_t tok = blk / nb, b = blk - tok * nb;
     const __amdgpu_buffer_rsrc_t r = make_rsrc(x, (nblocks / nb) * K * 4);
     const uint32_t o = blk < nblocks ? (tok * K + b * 32 + part * 4) * 4 : 0x80000000u;  // whole 8-lane groups
-    float f[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) f[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, o + 4 * e, 0, 0));
+    const v4u u = __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, 0);  // any dword alignment
+    const float f[4] = {__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w)};
     const uint32_t m = max8_u32(max(max(abs_key(f[0]), abs_key(f[1])), max(abs_key(f[2]), abs_key(f[3]))));
     float scale, inv;
     quant_params(__uint_as_float(m), scale, inv);
@@ -1364,9 +1366,8 @@ k_q8_act_quantize_bm(uint32_t nblocks, uint32_t nb, uint32_t K, uint32_t T4, uin
     const uint32_t tok = blk / nb, b = blk - tok * nb;
     const __amdgpu_buffer_rsrc_t r = make_rsrc(x, (nblocks / nb) * K * 4);
     const uint32_t o = blk < nblocks ? (tok * K + b * 32 + part * 4) * 4 : 0x80000000u;
-    float f[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) f[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, o + 4 * e, 0, 0));
+    const v4u u = __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, 0);  // any dword alignment
+    const float f[4] = {__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w)};
     const uint32_t m = max8_u32(max(max(abs_key(f[0]), abs_key(f[1])), max(abs_key(f[2]), abs_key(f[3]))));
     float scale, inv;
     quant_params(__uint_as_float(m), scale, inv);
@@ -1755,6 +1756,28 @@ int mma_mul_mat(uint32_t N, uint32_t nb, uint32_t K, uint32_t T, const float* x,
     return mma_launch<1, 2, 4, 2>(N, nb, T, W, workspace, dxo, y, s);
 }
 
+// Whether 5+ tokens go to the prompt kernel (q8_0_prompt.hip, 64 rows x 64
+// tokens per workgroup, one workgroup per CU at a time).
+//  * Rows of a part of 16 blocks, or not 16-byte aligned: always (the
+//    alternative is k_q8_0_mul_mat_g: 4096 x 11008 at 64 tokens 462 -> 45 us,
+//    at 8 tokens 63 -> 37, 1000 x 2080 at 100 tokens 140 -> 18).
+//  * More than 64 tokens: from one workgroup on every second CU (4096 x 4096 at
+//    96 / 128 / 512 tokens 24.0 / 30.1 / 100 -> 22.1 / 22.6 / 42 us; at 64
+//    workgroups, 2048 x 4096 at 128 tokens, 18.1 -> 22.3), but from one on
+//    every CU where the residue-split kernel shares a row group's K over four
+//    workgroups (4096 x 14336 at 128 tokens 50.4 -> 60.5, at 256 95 -> 64).
+//  * 33-64 tokens: one round of the CUs that is over half full (14336 x 8192
+//    at 64 tokens 63 -> 46, 11008 x 2048 18.8 -> 16.5; 8192 x 8192, half full,
+//    34.4 -> 37.8; 28672 x 4096, two rounds, 46 -> 50).
+bool prompt_wanted(uint32_t N, uint32_t nb, uint32_t T, bool rows16) {
+    if (!rows16) return true;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    const uint64_t cus = cu_count(dev), wgs = (uint64_t)((N + 63) / 64) * ((T + 63) / 64);
+    if (T > 64) return wgs >= (nb >= kMmrMinBlocks ? cus : cus / 2);
+    return T > 32 && wgs > cus / 2 && wgs <= cus;
+}
+
 // A K-quant GEMV on the streaming kernel: NW waves per workgroup, SB
 // super-blocks per item, SBF per item for matrices with few rows (4-wave
 // workgroups).  -1 when the rows are not 16-byte aligned or a partial
@@ -1936,6 +1959,16 @@ extern "C" int ane_hip_q8_0_mul_mat(uint32_t N, uint32_t K, uint32_t T, const fl
             r = T == 1 ? stream_auto<kModeG, 1, kFusePreQuant>(N, nb, K, T, xq, W, y, s)
                        : stream_auto<kModeG, kMaxStreamTokens, kFusePreQuant>(N, nb, K, T, xq, W, y, s);
         }
+        if (r >= 0) return r;
+    }
+    if (T > kMaxStreamTokens && prompt_eligible(N, nb, T, W) && (uint64_t)T * K * 4 < 0x80000000ull &&
+        prompt_wanted(N, nb, T, nb % kMmaSb == 0 && stream_eligible(N, nb, K, T, W))) {
+        const uint32_t Tp = (T + 15) / 16 * 16;
+        uint8_t* qxb = static_cast<uint8_t*>(workspace);
+        float* dxb;
+        const int st = quantize_bt(nb, K, T, Tp, x, qxb, &dxb, s);
+        if (st != ANE_OK) return st;
+        const int r = prompt_mul_mat(N, nb, T, W, qxb, dxb, Tp, y, s);
         if (r >= 0) return r;
     }
     if (T > kMaxStreamTokens && nb % kMmaSb == 0 && stream_eligible(N, nb, K, T, W)) {

@@ -84,9 +84,8 @@ k_q8_act_quantize_bt(uint32_t T, uint32_t Tp, uint32_t nb, uint32_t K, const flo
     const uint32_t tok = blk / nb, b = blk - tok * nb;
     const __amdgpu_buffer_rsrc_t r = make_rsrc(x, T * K * 4);
     const uint32_t o = tok < T ? (tok * K + b * 32 + part * 4) * 4 : 0x80000000u;
-    float f[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) f[e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, o + 4 * e, 0, 0));
+    const v4u u = __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, 0);  // any dword alignment
+    const float f[4] = {__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w)};
     const uint32_t m = max8_u32(max(max(abs_key(f[0]), abs_key(f[1])), max(abs_key(f[2]), abs_key(f[3]))));
     float scale, inv;
     quant_params(__uint_as_float(m), scale, inv);
@@ -413,6 +412,16 @@ uint64_t mmv_workspace_bound(uint32_t nb, uint32_t T) {
     return mmv_workspace_bytes(nb, pl);
 }
 
+int quantize_bt(uint32_t nb, uint32_t K, uint32_t T, uint32_t Tp, const float* x, uint8_t* qxb, float** dxb,
+                hipStream_t s) {
+    *dxb = reinterpret_cast<float*>(qxb + ceil_to((uint64_t)nb * Tp * 32, 256));
+    const uint32_t nthreads = nb * Tp * 8;
+    hipLaunchKernelGGL(k_q8_act_quantize_bt, dim3((nthreads + 255) / 256), dim3(256), 0, s, T, Tp, nb, K, x, qxb,
+                       *dxb);
+    ANE_HIP_CHECK_LAUNCH();
+    return ANE_OK;
+}
+
 int mmv_mul_mat(uint32_t N, uint32_t nb, uint32_t K, uint32_t T, const float* x, const void* W, float* y,
                 void* workspace, size_t workspace_bytes, hipStream_t s) {
     const MmvPlan pl = mmv_plan(N, nb, T);
@@ -422,11 +431,9 @@ int mmv_mul_mat(uint32_t N, uint32_t nb, uint32_t K, uint32_t T, const float* x,
         (uint64_t)T * K * 4 >= 0x80000000ull)
         return -1;
     uint8_t* qxb = static_cast<uint8_t*>(workspace);
-    float* dxb = reinterpret_cast<float*>(qxb + ceil_to((uint64_t)nb * pl.Tp * 32, 256));
-    const uint32_t nthreads = nb * pl.Tp * 8;
-    hipLaunchKernelGGL(k_q8_act_quantize_bt, dim3((nthreads + 255) / 256), dim3(256), 0, s, T, pl.Tp, nb, K, x, qxb,
-                       dxb);
-    ANE_HIP_CHECK_LAUNCH();
+    float* dxb;
+    const int st = quantize_bt(nb, K, T, pl.Tp, x, qxb, &dxb, s);
+    if (st != ANE_OK) return st;
     if (nb / 16 == 28) return mmv_launch<28, 1, 16>(N, T, pl.Tp, pl.n_tg, pl.rt_per_wg, W, qxb, dxb, y, s);
     if (pl.TT == 4) return mmv_launch<8, 4, 16>(N, T, pl.Tp, pl.n_tg, pl.rt_per_wg, W, qxb, dxb, y, s);
     if (pl.TT == 2) return mmv_launch<8, 2, 16>(N, T, pl.Tp, pl.n_tg, pl.rt_per_wg, W, qxb, dxb, y, s);

@@ -19,6 +19,10 @@ bool mmv_fills_cus(uint32_t N);
 uint64_t mmv_workspace_bytes(uint32_t nb, const MmvPlan& pl);
 // The same for any plan of T tokens (the activation form of ceil16(T) tokens).
 uint64_t mmv_workspace_bound(uint32_t nb, uint32_t T);
+// x quantized into the block-major activation form at qxb, its scales after
+// it (*dxb): mmv_workspace_bytes of a plan with Tp tokens.
+int quantize_bt(uint32_t nb, uint32_t K, uint32_t T, uint32_t Tp, const float* x, uint8_t* qxb, float** dxb,
+                hipStream_t s);
 // y[T x N] = the G-mode product of x[T x K] with N Q8_0 rows of nb blocks;
 // -1 when the shape or the workspace does not fit this kernel (nothing is
 // launched), else an ane_status.
