@@ -187,7 +187,7 @@ static int launch_gemm(const GemmParams& p, hipStream_t s) {
     if (p.Mout == 0 || p.Nout == 0) return ANE_OK;
     if (BL == kBTransposed && !AU8) {
         // 256-tiles while they fill every CU, few rows on the skinny kernel,
-        // otherwise 128-tiles (four times the workgroups)
+        // otherwise 128-tiles (four times the workgroups) or 64-tiles
         const uint64_t tiles256 = (uint64_t)((p.Mout + 255) / 256) * ((p.Nout + 255) / 256);
         const bool e256 = tile256_eligible(p);
         if (e256 && tiles256 >= tile256_min_tiles()) return launch_gemm_tile256(p, s);
@@ -195,6 +195,11 @@ static int launch_gemm(const GemmParams& p, hipStream_t s) {
         if (tile128_eligible(p)) {
             // one 128-tile per CU or fewer: the deeper ring; more: two per CU
             const uint64_t tiles128 = (uint64_t)((p.Mout + 127) / 128) * ((p.Nout + 127) / 128);
+            // 128-tiles on at most half of the CUs: 64-tiles (whole
+            // dense_fused_i8, 128- and 64-tiles: 301 x 2003 x 1777 24.4 / 20.0
+            // us, 1024 x 1024 x 4096 33.4 / 27.5, 256 x 4096 x 4096 47.0 / 41.0,
+            // 1000 x 1536 x 1000 19.2 / 17.7; raw int32 of 1024^3 11.6 / 12.2)
+            if (tiles128 * 2 <= tile256_min_tiles() && !p.Craw && tile64_eligible(p)) return launch_gemm_tile64(p, s);
             if (tiles128 <= tile256_min_tiles() && tile128d_eligible(p)) return launch_gemm_tile128d(p, s);
             return launch_gemm_tile128(p, s);
         }
@@ -379,24 +384,27 @@ static int fused_check(int32_t M, int32_t N, int32_t K, const void* workspace, s
     return ANE_OK;
 }
 
-extern "C" int ane_hip_dense_fused_i8_quantize(int32_t M, int32_t N, int32_t K, const float* A,
-                                               const float* B, float* scales_out, void* workspace,
-                                               size_t workspace_bytes, void* stream) {
+static int fused_quantize(int32_t M, int32_t N, int32_t K, const float* A, const float* B, float* scales_out,
+                          void* workspace, size_t workspace_bytes, bool whole_op, hipStream_t s) {
     int st = fused_check(M, N, K, workspace, workspace_bytes);
     if (st != ANE_OK) return st;
     if (M == 0 || N == 0) return ANE_OK;
     if (K > 0 && (!A || !B)) return ANE_ERR_BAD_POINTER;
-    hipStream_t s = (hipStream_t)stream;
     const FusedLayout L = fused_layout(M, N, K, workspace);
-    const uint64_t Kp = L.Kp;
-    st = launch_fused_quantize(A, B, (uint32_t)M, (uint32_t)N, (uint32_t)K, (uint32_t)Kp, L.partials,
-                               L.qA, L.qBt, L.scales, L.wstatus, s);
+    st = launch_fused_quantize(A, B, (uint32_t)M, (uint32_t)N, (uint32_t)K, (uint32_t)L.Kp, L.partials, L.qA, L.qBt,
+                               L.scales, L.wstatus, whole_op, s);
     if (st != ANE_OK) return st;
     if (scales_out) {
         hipError_t e = hipMemcpyAsync(scales_out, L.scales, 2 * sizeof(float), hipMemcpyDeviceToDevice, s);
         if (e != hipSuccess) return ANE_ERR_HIP;
     }
     return ANE_OK;
+}
+
+extern "C" int ane_hip_dense_fused_i8_quantize(int32_t M, int32_t N, int32_t K, const float* A,
+                                               const float* B, float* scales_out, void* workspace,
+                                               size_t workspace_bytes, void* stream) {
+    return fused_quantize(M, N, K, A, B, scales_out, workspace, workspace_bytes, false, (hipStream_t)stream);
 }
 
 extern "C" int ane_hip_dense_fused_i8_gemm(int32_t M, int32_t N, int32_t K, float scale, int relu,
@@ -485,8 +493,7 @@ extern "C" int ane_hip_dense_fused_i8(int32_t M, int32_t N, int32_t K, float sca
             return ANE_OK;
         }
     }
-    int st = ane_hip_dense_fused_i8_quantize(M, N, K, A, B, scales_out, workspace, workspace_bytes,
-                                             stream);
+    int st = fused_quantize(M, N, K, A, B, scales_out, workspace, workspace_bytes, true, (hipStream_t)stream);
     if (st != ANE_OK) return st;
     return ane_hip_dense_fused_i8_gemm(M, N, K, scale, relu, C, workspace, workspace_bytes, stream);
 }

@@ -33,7 +33,7 @@ struct GemmParams {
 constexpr uint32_t kFusedPartials = 1024;
 int launch_fused_quantize(const float* A, const float* B, uint32_t M, uint32_t N, uint32_t K,
                           uint32_t Kp, uint32_t* partials, int8_t* qA, int8_t* qBt, float* scales,
-                          uint32_t* wstatus, hipStream_t s);
+                          uint32_t* wstatus, bool whole_op, hipStream_t s);
 // The whole of dense_fused_i8 for small operands (K <= 1024, at most 512
 // tiles of 16 x 16): the absmax pass, then one launch that quantizes each tile's rows
 // and columns into LDS and contracts them (quantize_fused.hip).  Writes C,
@@ -75,6 +75,10 @@ int launch_gemm_tile128(const GemmParams& p, hipStream_t s, uint32_t ksplit = 1)
 // per CU (gemm_i8_tile128d.hip): for launches of at most one workgroup per CU.
 bool tile128d_eligible(const GemmParams& p, bool any_rows = false);
 int launch_gemm_tile128d(const GemmParams& p, hipStream_t s, uint32_t ksplit = 1);
+
+// The same at 64 x 64 tiles (gemm_i8_tile64.hip).
+bool tile64_eligible(const GemmParams& p, bool any_rows = false);
+int launch_gemm_tile64(const GemmParams& p, hipStream_t s, uint32_t ksplit = 1);
 
 // The same loop with B in SMOPA panels (ldb = Kp / 4 groups of 64 bytes per
 // panel) and A int8 or uint8, at 256 x 256 (gemm_i8_panel256.hip) and 128 x

@@ -70,8 +70,12 @@ namespace {
 #ifndef ANE_TILE_WAVES
 #define ANE_TILE_WAVES 4
 #endif
+#elif ANE_TILE == 64
+#ifndef ANE_TILE_WAVES
+#define ANE_TILE_WAVES 4
+#endif
 #else
-#error "ANE_TILE is 256 or 128"
+#error "ANE_TILE is 256, 128 or 64"
 #endif
 // ANE_TILE_STAGES: LDS ring depth (2 by default).  Slice kt+STAGES-1 is
 // copied while slice kt is multiplied, so STAGES-1 slices are in flight.
@@ -184,7 +188,8 @@ __device__ __forceinline__ void slice_pinned(v16i (&acc)[FM][FN], Frags& f0, Fra
                                              const uint32_t (&offB)[kDmaPerWave],
                                              const uint32_t (&kofs)[kDmaPerWave], int amask, Extra&& extra) {
     constexpr int nM = FM * FN, nD = FM + FN;
-    constexpr int kCopySteps = kPanel ? 1 : 2;          // k-steps that carry the copies
+    // k-steps that carry the copies: as few as leave an MFMA for each
+    constexpr int kCopySteps = kPanel ? 1 : nM == 1 ? kCopies : 2;
     constexpr int kPerStep = kCopies / kCopySteps;
     constexpr int kStride = nM / kPerStep;              // MFMAs per copy
     static_assert(kPerStep * kCopySteps == kCopies && kStride * kPerStep == nM && kCopySteps <= kSteps,

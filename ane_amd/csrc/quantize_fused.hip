@@ -34,6 +34,15 @@ __device__ __forceinline__ uint32_t absmax4(float4 v) {
     return umax(umax(abs_key(v.x), abs_key(v.y)), umax(abs_key(v.z), abs_key(v.w)));
 }
 
+// Four floats in one 16-byte load that needs no more than a float's
+// alignment: rows of a K or N that is not a multiple of four (2003 columns:
+// the quantize pass of 301 x 2003 x 1777 12.3 -> 7.3 us against single loads).
+__device__ __forceinline__ float4 load4(const float* p) {
+    float4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+
 // Pass 1: blocks [0, nbA) reduce A, [nbA, nbA+nbB) reduce B.  Each block
 // reads one contiguous range of its tensor's float4s (contiguous ranges per
 // workgroup measured faster on this HBM than a grid-stride interleave),
@@ -105,7 +114,6 @@ k_quantize_two(const float* __restrict__ A, const float* __restrict__ B, uint32_
     if (isA) {
         const uint64_t chunks_per_row = Kp / 16;
         const uint64_t total = (uint64_t)M * chunks_per_row;
-        const bool vec = ((K & 3) == 0) && ((((uintptr_t)A) & 15) == 0);
         // one contiguous range of chunks per block
         const uint64_t per = (total + nqA - 1) / nqA;
         const uint64_t c0 = (uint64_t)blockIdx.x * per, c1 = c0 + per < total ? c0 + per : total;
@@ -114,11 +122,8 @@ k_quantize_two(const float* __restrict__ A, const float* __restrict__ B, uint32_
             const uint32_t k = (uint32_t)(c % chunks_per_row) * 16;
             const float* src = A + i * K + k;
             uint32_t w[4] = {0, 0, 0, 0};
-            if (vec && k + 16 <= K) {
-                const float4 v0 = reinterpret_cast<const float4*>(src)[0];
-                const float4 v1 = reinterpret_cast<const float4*>(src)[1];
-                const float4 v2 = reinterpret_cast<const float4*>(src)[2];
-                const float4 v3 = reinterpret_cast<const float4*>(src)[3];
+            if (k + 16 <= K) {
+                const float4 v0 = load4(src), v1 = load4(src + 4), v2 = load4(src + 8), v3 = load4(src + 12);
                 if (fast) {
                     w[0] = pack4_fast(v0.x, v0.y, v0.z, v0.w, inv);
                     w[1] = pack4_fast(v1.x, v1.y, v1.z, v1.w, inv);
@@ -144,7 +149,7 @@ k_quantize_two(const float* __restrict__ A, const float* __restrict__ B, uint32_
     const uint32_t k0 = (tb / ntn) * kBTK, n0 = (tb % ntn) * kBTN;
     const uint32_t kq = threadIdx.x >> 4, nq = threadIdx.x & 15;
     const uint32_t gn = n0 + 4 * nq;
-    const bool vec = ((N & 3) == 0) && ((((uintptr_t)B) & 15) == 0) && gn + 3 < N;
+    const bool vec = gn + 3 < N;
 #pragma unroll
     for (int g = 0; g < 2; g++) {
         float v[4][4];
@@ -152,7 +157,7 @@ k_quantize_two(const float* __restrict__ A, const float* __restrict__ B, uint32_
         for (int i = 0; i < 4; i++) {
             const uint32_t gk = k0 + g * 64 + 4 * kq + i;
             if (gk < K && vec) {
-                const float4 f = *reinterpret_cast<const float4*>(B + (uint64_t)gk * N + gn);
+                const float4 f = load4(B + (uint64_t)gk * N + gn);
                 v[i][0] = f.x; v[i][1] = f.y; v[i][2] = f.z; v[i][3] = f.w;
             } else {
 #pragma unroll
@@ -345,6 +350,7 @@ static_assert(kRLdsA4 % kWave == 0, "the LDS part of A is copied in whole 64-slo
 static_assert(kRNT * kTileDw * 4 <= kRLdsA4 * 16, "the B transposes fit in A's LDS");
 constexpr uint64_t kSyncTimeoutTicks = 200000000ull;  // 2 s at 100 MHz
 constexpr uint64_t kResidentMinBytes = (uint64_t)12 << 20;
+constexpr uint64_t kEagerResidentMinBytes = (uint64_t)112 << 20;
 
 // Grid-wide exchange of the workgroup maxima, by thread 0 of each
 // workgroup.  Every access is an agent-scope atomic (coherent across the
@@ -959,6 +965,10 @@ struct ResidentDevice {
     hipEvent_t last = nullptr;
     hipStream_t last_stream = nullptr;
     bool last_valid = false;
+    // The stream of the last uncaptured call that a grid-wide-wait kernel fits,
+    // whichever route it took: such a kernel is captured on that stream only.
+    hipStream_t call_stream = nullptr;
+    bool call_valid = false;
     uint32_t tag = 0;  // the last launch's tag (launches are numbered from 1)
 };
 std::mutex g_res_mu;
@@ -1009,11 +1019,12 @@ ResidentDevice* resident_device(hipStream_t s, int* dev_out) {
 // of such launches per device, the launch tag and the choice of a
 // cooperative launch.  `fits(G)` checks the shape against the kernel's grid
 // G (d.*grid_of); `go(G, sync, tag, limit, coop)` queues the kernel and
-// returns the launch call's error.  Returns true when the kernel was queued
+// returns the launch call's error.  eager: whether the kernel is taken outside
+// capture.  Returns true when the kernel was queued
 // (*status = ANE_ERR_HIP if it failed after that), false when the route
 // cannot run (nothing queued: the caller takes another route).
 template <class Fits, class Go>
-bool launch_grid_wait(hipStream_t s, uint32_t ResidentDevice::*grid_of, Fits fits, Go go, int* status) {
+bool launch_grid_wait(hipStream_t s, uint32_t ResidentDevice::*grid_of, bool eager, Fits fits, Go go, int* status) {
     *status = ANE_OK;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
@@ -1028,13 +1039,18 @@ bool launch_grid_wait(hipStream_t s, uint32_t ResidentDevice::*grid_of, Fits fit
     ResidentDevice& d = *dp;
     const uint32_t G = d.*grid_of;
     if (!G || !fits(G)) return false;
+    if (!capturing && !eager) {
+        d.call_stream = s;
+        d.call_valid = true;
+        return false;
+    }
     // Grid-wide-wait launches on one device are ordered: a launch on another
     // stream than the previous one waits for it.  A captured launch cannot
     // wait for work outside its graph, so under capture the route is taken
     // only on the stream of the previous launch (graph replays are ordered
     // by their caller).
     const bool other = d.last_valid && d.last_stream != s;
-    if (capturing && other) return false;
+    if (capturing && (other || (d.call_valid && d.call_stream != s))) return false;
     if (!capturing) {
         if (!d.last && hipEventCreateWithFlags(&d.last, hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
@@ -1064,8 +1080,8 @@ bool launch_grid_wait(hipStream_t s, uint32_t ResidentDevice::*grid_of, Fits fit
             *status = ANE_ERR_HIP;
             return true;
         }
-        d.last_stream = s;
-        d.last_valid = true;
+        d.last_stream = d.call_stream = s;
+        d.last_valid = d.call_valid = true;
     }
     return true;
 }
@@ -1075,7 +1091,7 @@ bool launch_grid_wait(hipStream_t s, uint32_t ResidentDevice::*grid_of, Fits fit
 // B tiles per workgroup.  Returns true when it launched.
 bool launch_resident(const float* A, const float* B, uint32_t M, uint32_t N, uint32_t K,
                      uint32_t* partials, int8_t* qA, int8_t* qBt, float* scales, uint32_t* wstatus,
-                     hipStream_t s, int* status) {
+                     bool whole_op, hipStream_t s, int* status) {
     *status = ANE_OK;
     if (K == 0 || M == 0 || N == 0 || (K % kBTK) || (N % kBTN)) return false;
     // below ~12 MiB of operands the two launches of the two-pass route are
@@ -1115,7 +1131,14 @@ bool launch_resident(const float* A, const float* B, uint32_t M, uint32_t N, uin
                            kPerT, kPartials, kQA, kQBt, kScales, kSync, kTag, kLimit, kStatus);
         return hipGetLastError();
     };
-    return launch_grid_wait(s, &ResidentDevice::grid, fits, go, status);
+    // Outside capture the launch is cooperative, which costs 15-20 us more of the
+    // stream's time than a plain one, so the two-pass route (no wait) is taken
+    // there while a second read of the operands costs less than that: cooperative
+    // against two-pass 2048^3 53.0 / 30.7 us, 512 x 512 x 4096 48.8 / 22.8, 128 x
+    // 4096 x 4096 55.8 / 41.4, 1024 x 4096 x 4096 72.0 / 59.5, 4096^3 129.4 / 131.
+    const bool eager = !whole_op || !cooperative_launches() ||
+                       ((uint64_t)M * K + (uint64_t)K * N) * 4 >= kEagerResidentMinBytes;
+    return launch_grid_wait(s, &ResidentDevice::grid, eager, fits, go, status);
 }
 
 // The current device's slot, if the resident route was ever set up on it.
@@ -1137,9 +1160,9 @@ uint32_t blocks_for(uint64_t n) {
 
 int launch_fused_quantize(const float* A, const float* B, uint32_t M, uint32_t N, uint32_t K,
                           uint32_t Kp, uint32_t* partials, int8_t* qA, int8_t* qBt, float* scales,
-                          uint32_t* wstatus, hipStream_t s) {
+                          uint32_t* wstatus, bool whole_op, hipStream_t s) {
     int st = ANE_OK;
-    if (Kp == K && launch_resident(A, B, M, N, K, partials, qA, qBt, scales, wstatus, s, &st)) return st;
+    if (Kp == K && launch_resident(A, B, M, N, K, partials, qA, qBt, scales, wstatus, whole_op, s, &st)) return st;
     const uint64_t nA = (uint64_t)M * K, nB = (uint64_t)K * N;
     const uint32_t nbA = blocks_for(nA), nbB = blocks_for(nB);
     hipLaunchKernelGGL(k_absmax_two, dim3(nbA + nbB), dim3(kT), 0, s, A, nA, nbA, B, nB, nbB, partials);
@@ -1216,7 +1239,7 @@ bool launch_fused_strip(const float* A, const float* B, uint32_t M, uint32_t N, 
                            kPartials, kScales, kSync, kTag, kLimit, kStatus);
         return hipGetLastError();
     };
-    return launch_grid_wait(s, &ResidentDevice::grid_strip, fits, go, status);
+    return launch_grid_wait(s, &ResidentDevice::grid_strip, true, fits, go, status);
 }
 
 }  // namespace ane
