@@ -153,6 +153,9 @@ k_gemm_i8(GemmParams p) {
                 if (AU8) v = (int32_t)((uint32_t)v + 128u * (uint32_t)colsum[ni]);
                 if (p.Craw) {
                     p.Craw[(uint64_t)i * p.ldc + j] = v;
+                } else if (p.ig) {
+                    p.C[(uint64_t)i * p.ldc + j] =
+                        ig_out(p, v, ig_sum(p.igc, p.nsum, p.Nout, j), ig_sum(p.igr, p.nsum, p.Mout, i));
                 } else {
                     float f = __fadd_rn(__fmul_rn((float)v, s), bj);
                     p.C[(uint64_t)i * p.ldc + j] = fmax_a(f, p.lo);
@@ -222,6 +225,8 @@ static int launch_gemm(const GemmParams& p, hipStream_t s) {
     ANE_HIP_CHECK_LAUNCH();
     return ANE_OK;
 }
+
+int launch_gemm_rows(const GemmParams& p, hipStream_t s) { return launch_gemm<kBTransposed, false>(p, s); }
 
 static bool aligned16(const void* ptr) { return (((uintptr_t)ptr) & 15) == 0; }
 

@@ -22,7 +22,30 @@ struct GemmParams {
     float* C;             // fp32 output, row stride ldc
     uint64_t ldc;
     int32_t* Craw;        // raw int32 output instead (debug entry)
+    // Integer GEMM epilogue (igemm.hip) instead of the one above: C =
+    // fl((float)(acc + 128 colsum[j] + 128 rowsum[i] + corr) * s), the sums given
+    // as partials of nsum runs of K (colsum[p * Nout + j], rowsum[p * Mout + i];
+    // null: none).
+    bool ig;
+    const int32_t* igc;
+    const int32_t* igr;
+    uint32_t nsum, corr;
 };
+
+// Sum of the partials of column or row x (n columns or rows in all); 0 without.
+__device__ __forceinline__ uint32_t ig_sum(const int32_t* part, uint32_t nsum, uint32_t n, uint32_t x) {
+    uint32_t t = 0;
+    if (part)
+        for (uint32_t p = 0; p < nsum; p++) t += (uint32_t)part[(uint64_t)p * n + (x < n ? x : n - 1)];
+    return 128u * t;
+}
+__device__ __forceinline__ float ig_out(const GemmParams& p, int32_t acc, uint32_t col, uint32_t row) {
+    return __fmul_rn((float)(int32_t)((uint32_t)acc + col + row + p.corr), p.s);
+}
+
+// The contraction with any of the epilogues on signed rows of A and Bt
+// (gemm_i8.hip chooses the kernel).
+int launch_gemm_rows(const GemmParams& p, hipStream_t s);
 
 // dense_fused_i8 operand preparation (quantize_fused.hip): absmax partials
 // (kFusedPartials per tensor), qA (M x Kp), qBt (N x Kp), scales {sa, sb},

@@ -126,6 +126,7 @@ __global__ void __launch_bounds__(256) k_gemm_skinny(GemmParams p) {
     if (p.sdev) s = __fmul_rn(__fmul_rn(p.sdev[0], p.sdev[1]), p.smul);
     const uint32_t j = n0 + c16;
     const float bj = (p.bias && j < p.Nout) ? p.bias[j] : 0.0f;
+    const uint32_t igc = p.ig ? ig_sum(p.igc, p.nsum, p.Nout, j) : 0u;
     for (uint32_t r = wave; r < (uint32_t)MB; r += 4) {
         v4i t = red[0][r][lane] + red[1][r][lane] + red[2][r][lane] + red[3][r][lane];
         if (AU8)
@@ -137,6 +138,8 @@ __global__ void __launch_bounds__(256) k_gemm_skinny(GemmParams p) {
             if (row >= p.Mout || j >= p.Nout) continue;
             if (p.Craw) {
                 p.Craw[(uint64_t)row * p.ldc + j] = t[i];
+            } else if (p.ig) {
+                p.C[(uint64_t)row * p.ldc + j] = ig_out(p, t[i], igc, ig_sum(p.igr, p.nsum, p.Mout, row));
             } else {
                 const float f = __fadd_rn(__fmul_rn((float)t[i], s), bj);
                 p.C[(uint64_t)row * p.ldc + j] = fmax_a(f, p.lo);
