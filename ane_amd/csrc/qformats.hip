@@ -31,7 +31,12 @@ namespace {
 
 using namespace qf;
 
-constexpr uint32_t kXChunk = 4096;  // x values staged per pass (16 KB of LDS: five workgroups per CU)
+// x values staged per pass: 16 KB of LDS, five workgroups of 16 rows per CU;
+// 8-row workgroups take half of that, so that seven fit (with 16 KB each,
+// 14336 rows of Q6_K measured no faster than 16-row workgroups; with 8 KB
+// everywhere 4096 rows 11.7 -> 12.2 us)
+template <int RW>
+constexpr uint32_t kXValues = RW == 8 ? 2048 : 4096;
 
 template <class F>
 struct Stage {
@@ -47,6 +52,7 @@ k_qgemv(uint32_t M, uint32_t nsb, uint32_t K, const float* __restrict__ x, const
         uint32_t wbytes, float* __restrict__ y) {
     // K here is nsb * values: the x staging below never reads past it
     using St = Stage<F>;
+    constexpr uint32_t kXChunk = kXValues<RW>;
     // windows 64 bytes apart beyond their length: the four rows of a wave
     // read their bytes from four different bank groups
     __shared__ __attribute__((aligned(16))) uint8_t win_all[RW][St::kWindow + 64];
@@ -163,8 +169,9 @@ int qgemv_launch(uint32_t M, uint32_t K, const float* x, const void* W, float* y
     const uint32_t range = (uint32_t)((off + (uint64_t)M * nsb * F::kBytes + 3) & ~(uint64_t)3);
     // 16 rows per workgroup from one workgroup per CU up (4096 rows on 256
     // CUs: 8 rows per workgroup measured slower there, the x staging then
-    // serving half as many rows), 8 or 4 below that so short matrices still
-    // spread over the CUs
+    // serving half as many rows) unless 8 spread the rows more evenly over the
+    // CUs (14336 rows: 56 per CU at most, not 64; Q6_K 26.7 -> 25.2 us), 8 or 4
+    // below that so short matrices still spread over the CUs
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return ANE_ERR_HIP;
     int cus = 0;
@@ -175,9 +182,10 @@ int qgemv_launch(uint32_t M, uint32_t K, const float* x, const void* W, float* y
     // x is staged only up to the values the super-blocks consume: a
     // remainder of K past them is never read (the caller's x may end there)
     const uint32_t kx = nsb * F::kValues;
-    if (M >= 16u * (uint32_t)cus)
+    const uint64_t c = (uint64_t)cus, per16 = (M + 16 * c - 1) / (16 * c) * 16, per8 = (M + 8 * c - 1) / (8 * c) * 8;
+    if (M >= 16 * c && per16 <= per8)
         hipLaunchKernelGGL((k_qgemv<F, 16>), dim3((M + 15) / 16), dim3(256), 0, s, M, nsb, kx, x, base, off, range, y);
-    else if (M >= 8u * (uint32_t)cus)
+    else if (M >= 8 * c)
         hipLaunchKernelGGL((k_qgemv<F, 8>), dim3((M + 7) / 8), dim3(128), 0, s, M, nsb, kx, x, base, off, range, y);
     else
         hipLaunchKernelGGL((k_qgemv<F, 4>), dim3((M + 3) / 4), dim3(64), 0, s, M, nsb, kx, x, base, off, range, y);
