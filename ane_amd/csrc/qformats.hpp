@@ -34,8 +34,11 @@ __device__ __forceinline__ uint32_t fld32(const uint8_t* p) {
     if constexpr (A >= 4) {
         return *reinterpret_cast<const uint32_t*>(p);
     } else if constexpr (A == 2) {
-        return (uint32_t)*reinterpret_cast<const uint16_t*>(p) |
-               ((uint32_t)*reinterpret_cast<const uint16_t*>(p + 2) << 16);
+        // (the empty asm keeps the compiler from fusing the two reads into one
+        // 32-bit read, which has no alias information either)
+        uint32_t hi = *reinterpret_cast<const uint16_t*>(p + 2);
+        asm("" : "+v"(hi));
+        return (uint32_t)*reinterpret_cast<const uint16_t*>(p) | (hi << 16);
     } else {
         return lu32(p);
     }
