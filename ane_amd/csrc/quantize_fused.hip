@@ -965,10 +965,6 @@ struct ResidentDevice {
     hipEvent_t last = nullptr;
     hipStream_t last_stream = nullptr;
     bool last_valid = false;
-    // The stream of the last uncaptured call that a grid-wide-wait kernel fits,
-    // whichever route it took: such a kernel is captured on that stream only.
-    hipStream_t call_stream = nullptr;
-    bool call_valid = false;
     uint32_t tag = 0;  // the last launch's tag (launches are numbered from 1)
 };
 std::mutex g_res_mu;
@@ -1039,18 +1035,15 @@ bool launch_grid_wait(hipStream_t s, uint32_t ResidentDevice::*grid_of, bool eag
     ResidentDevice& d = *dp;
     const uint32_t G = d.*grid_of;
     if (!G || !fits(G)) return false;
-    if (!capturing && !eager) {
-        d.call_stream = s;
-        d.call_valid = true;
-        return false;
-    }
     // Grid-wide-wait launches on one device are ordered: a launch on another
     // stream than the previous one waits for it.  A captured launch cannot
     // wait for work outside its graph, so under capture the route is taken
     // only on the stream of the previous launch (graph replays are ordered
-    // by their caller).
+    // by their caller).  An uncaptured call that the kernel fits but that takes
+    // another route is ordered the same way, so that it too makes its stream
+    // the one to capture on.
     const bool other = d.last_valid && d.last_stream != s;
-    if (capturing && (other || (d.call_valid && d.call_stream != s))) return false;
+    if (capturing && other) return false;
     if (!capturing) {
         if (!d.last && hipEventCreateWithFlags(&d.last, hipEventDisableTiming) != hipSuccess) {
             (void)hipGetLastError();
@@ -1059,6 +1052,16 @@ bool launch_grid_wait(hipStream_t s, uint32_t ResidentDevice::*grid_of, bool eag
         }
         if (other && hipStreamWaitEvent(s, d.last, 0) != hipSuccess) {
             (void)hipGetLastError();
+            return false;
+        }
+        if (!eager) {
+            // recorded behind that wait, the event still covers the launch before
+            if ((other || !d.last_valid) && hipEventRecord(d.last, s) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
+            d.last_stream = s;
+            d.last_valid = true;
             return false;
         }
     }
@@ -1080,8 +1083,8 @@ bool launch_grid_wait(hipStream_t s, uint32_t ResidentDevice::*grid_of, bool eag
             *status = ANE_ERR_HIP;
             return true;
         }
-        d.last_stream = d.call_stream = s;
-        d.last_valid = d.call_valid = true;
+        d.last_stream = s;
+        d.last_valid = true;
     }
     return true;
 }

@@ -60,3 +60,33 @@ def test_capture_follows_the_last_eager_stream(ane, oracle):
             count = int(host(ws[256 + 8192:256 + 8196]).view(np.uint32)[0])
             assert (count > 0) == waits
         del g
+
+
+def test_capture_after_a_wait_on_another_stream(ane, oracle):
+    """A kernel with a grid-wide wait ran on s1 (16 x 4096 x 4096, taken eagerly
+    too); an uncaptured 256 x 2048 x 2048 on s2, which takes the two-pass route,
+    makes s2 the stream to capture on: the captured call keeps its wait."""
+    import torch
+
+    M, N, K = 256, 2048, 2048
+    A, B = data.gemm_inputs(M, N, K, seed=37)
+    want = oracle.dense_fused_i8(M, N, K, F32(1.0), True, A, B)
+    dA, dB, C = dev(A), dev(B), torch.zeros(M * N, device="cuda")
+    ws = torch.empty(ane.dense_fused_i8_workspace_size(M, N, K), dtype=torch.uint8, device="cuda")
+    x, w, y = (torch.randn(n, device="cuda") for n in (16 * 4096, 4096 * 4096, 16 * 4096))
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    ane.dense_fused_i8(16, 4096, 4096, 1.0, True, x, w, y, stream=s1)
+    ane.dense_fused_i8(M, N, K, 1.0, True, dA, dB, C, workspace=ws, stream=s2)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s2):
+        ane.dense_fused_i8(M, N, K, 1.0, True, dA, dB, C, workspace=ws, stream=s2, check_wait=False)
+    for _ in range(3):
+        C.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        ane.dense_fused_i8_status(ws, stream=s2)
+        assert_same(host(C).reshape(M, N), want)
+        assert int(host(ws[256 + 8192:256 + 8196]).view(np.uint32)[0]) > 0
