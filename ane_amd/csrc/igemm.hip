@@ -29,8 +29,8 @@
 // which is exact modulo 2^32, like the handler's own wrapping sums.  Each tile
 // writes its rows' partial sums, added up in the epilogue (no atomics, nothing
 // to clear).  Signed operands that are already K-contiguous rows (A without
-// transA, B with transB) with 16-byte aligned rows skip the pre-pass: the
-// contraction reads them in place.  With beta = 0 the contraction writes C
+// transA, B with transB) with 16-byte aligned rows that C does not overlap skip
+// the pre-pass: the contraction reads them in place.  With beta = 0 the contraction writes C
 // itself; otherwise it leaves int32 sums and k_igemm_epilogue reads C.
 // Measured, 1536 x 2048 x 2048 uint8 x int8, both row-major: 27.4 -> 17.6 us
 // (byte loads into 64 x 64 tiles with atomic row sums, a fill, two gathers and
@@ -238,8 +238,17 @@ extern "C" int ane_hip_cblas_igemm(int variant, int semantics, uint8_t flags, ui
         // Signed operands already in the contraction's layout (A's rows, or
         // B's rows under transB, K contiguous with 16-byte aligned rows) are
         // read in place: no gather pass, no row sums needed (both signed).
-        const bool a_direct = !au && !bu && !ta && (lda & 15) == 0 && lda >= Ke && (((uintptr_t)A) & 15) == 0;
-        const bool b_direct = !au && !bu && tb && (ldb & 15) == 0 && ldb >= Ke && (((uintptr_t)B) & 15) == 0;
+        // Not where the contraction would write C over bytes that its other
+        // workgroups still read: an operand that overlaps C is gathered.
+        const uint64_t c_end = ((uint64_t)(M - 1) * ldc + N) * 4;
+        auto under_c = [&](const void* p, uint32_t rows, uint32_t ld) {
+            const uintptr_t x = (uintptr_t)p, c = (uintptr_t)C;
+            return !reads_c && x < c + c_end && c < x + (uint64_t)(rows - 1) * ld + Ke;
+        };
+        const bool a_direct = !au && !bu && !ta && (lda & 15) == 0 && lda >= Ke && (((uintptr_t)A) & 15) == 0 &&
+                              !under_c(A, M, lda);
+        const bool b_direct = !au && !bu && tb && (ldb & 15) == 0 && ldb >= Ke && (((uintptr_t)B) & 15) == 0 &&
+                              !under_c(B, N, ldb);
         // A rows: plain, the handler's transA addressing, or A^T (BLAS); Bt
         // rows: B^T of a K x N matrix, or B itself (transB)
         Gather ga = gather_of(M, Ke, A, !ta ? (int64_t)lda : 1, (ta && semantics == 0) ? (int64_t)lda - 1 : 0,

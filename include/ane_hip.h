@@ -235,7 +235,8 @@ int ane_hip_gemm_s8_i32(uint32_t M, uint32_t N, uint32_t K, const int8_t* A,
  * runs for the opcodes.  ANE_IGEMM_BLAS computes the documented form instead:
  * op(A) = A^T (A is K x M, stride lda) with transA, and
  * C = fl(fl(fl32(acc) * alpha) + fl(beta * C)), C not read when beta == 0.
- * Accumulation wraps modulo 2^32 in both. */
+ * Accumulation wraps modulo 2^32 in both.  On device buffers C may
+ * overlap A or B: operands are read as they were before the call. */
 #define ANE_IGEMM_SIGNED 0
 #define ANE_IGEMM_UNSIGNED 1
 #define ANE_IGEMM_MIXED 2

@@ -35,3 +35,29 @@ def test_tiles_and_sums(ane, oracle, kind, flags, M, N, K):
         kb, pb = at_offset(B, 3)
         ane.cblas_igemm(kind, flags, M, N, K, lda, ldb, N + 1, -1.5, beta, pa, pb, Cd, blas=bool(sem))
         assert_same(host(Cd), want)
+
+
+@pytest.mark.parametrize("which,flags", [("A", 0), ("A", 1), ("B", 2), ("B", 0)])
+@pytest.mark.parametrize("M,N,K,at", [(300, 700, 512, 0), (300, 700, 512, 160000), (40, 64, 128, 48), (500, 900, 320, 16)])
+def test_c_over_an_operand(ane, oracle, which, flags, M, N, K, at):
+    """igemm with beta = 0 whose C covers A or B (from byte `at` of C on): the
+    operand is read whole before C is written, also where it could be read in
+    place (A without transA, B with transB)."""
+    import torch
+
+    lda, ldb, ldc = (K if not flags & 1 else M + 16), (N if not flags & 2 else K + 16), N + 4
+    if flags & 1:
+        lda = -(-max(lda, K) // 16) * 16
+    A, B, C = _igemm_case("igemm", flags, M, N, K, lda, ldb, ldc, seed=M + N + K + flags)
+    for sem in (0, 1):
+        if flags & 1 and sem == 1:
+            A = np.resize(A, K * lda)
+        want = oracle.cblas_igemm(0, flags, M, N, K, lda, ldb, ldc, 0.5, 0.0, A, B, np.zeros_like(C), semantics=sem)
+        over = A if which == "A" else B
+        buf = torch.zeros(max(M * ldc * 4, at + over.size), dtype=torch.uint8, device="cuda")
+        buf[at:at + over.size] = dev(over.view(np.uint8))
+        a = buf.data_ptr() + at if which == "A" else dev(A)
+        b = buf.data_ptr() + at if which == "B" else dev(B)
+        ane.cblas_igemm("igemm", flags, M, N, K, lda, ldb, ldc, 0.5, 0.0, a, b, buf, blas=bool(sem))
+        got = host(buf)[:M * ldc * 4].view(F32).reshape(M, ldc)
+        assert_same(got[:, :N], np.asarray(want).reshape(M, ldc)[:, :N])
