@@ -292,6 +292,10 @@ int run(uint32_t N, uint32_t nb, uint32_t T, const float* x, const void* W, floa
     if (nb == 0 || (wp & 1) || (((uintptr_t)x) & 3) || wbytes + 2 * kMaxP * F::kBytes + 16 >= kOob ||
         ((uint64_t)T + 64) * nb * 128 + 2 * kMaxP * 128 >= kOob)
         return -1;
+    // Token t's y may take the place of an earlier token's x in the one launch
+    // per token; here every token is read and written at once.
+    const uintptr_t xp = (uintptr_t)x, yp = (uintptr_t)y;
+    if (xp < yp + (uint64_t)T * N * 4 && yp < xp + (uint64_t)T * nb * 128) return -1;
     // whole dwords: the range check drops a dword that crosses the end
     const uint32_t wrange = (uint32_t)((wbytes + 3) & ~(uint64_t)3);
     const uint8_t* Wa = reinterpret_cast<const uint8_t*>(wp - off);

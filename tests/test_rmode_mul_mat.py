@@ -72,3 +72,25 @@ def test_odd_weights_address_takes_the_gemv(ane, oracle):
     x = data.activations(T, K, seed=9)
     keep, Wd = weights_at(W, 7)
     assert_same(run_node(ane, True, N, K, T, Wd, dev(x)), want(oracle, True, N, K, W, x))
+
+
+@pytest.mark.parametrize("q4", [True, False])
+@pytest.mark.parametrize("K,T", [(64, 3), (256, 40)])
+def test_outputs_over_earlier_inputs(ane, oracle, q4, K, T):
+    """y one row before x in one buffer: token t's outputs replace token
+    t-1's inputs, and each token still sees its own (one GEMV per token)."""
+    import torch
+
+    W = data.q_weights("q4_0", K, K, seed=K) if q4 else data.q8_0_weights(K, K, seed=K)
+    x = data.activations(T, K, seed=T)
+    keep, Wd = weights_at(W, 0)
+    buf = torch.zeros((T + 1, K), device="cuda")
+    buf[1:].copy_(dev(x))
+    a = ane.ggml_tensor(ane.GgmlType.Q4_0 if q4 else ane.GgmlType.Q8_0, [K, K], Wd)
+    b = ane.ggml_tensor(ane.GgmlType.F32, [K, T], buf[1:])
+    d = ane.ggml_tensor(ane.GgmlType.F32, [K, T], buf[:T], op=ane.GgmlOp.MUL_MAT, src=(a, b))
+    be = ane.GgmlBackend(q8_mode=1)
+    be.compute(d)
+    got = host(buf)[:T]
+    be.close()
+    assert_same(got, want(oracle, q4, K, K, W, x))
