@@ -87,6 +87,10 @@ __host__ __device__ inline uint64_t ceil_to(uint64_t x, uint64_t m) {
     return (x + m - 1) / m * m;
 }
 
+// A dimension of a launch holds fewer than 2^32 work items (the runtime refuses
+// more); kernels for which a shape may pass that leave it to another route.
+inline bool launch_fits(uint64_t blocks, uint32_t threads) { return blocks * threads < (1ull << 32); }
+
 // ------------------------------------------------- DPP row permutations
 // v_mov_b32 with a DPP control: every lane reads the named lane of its own
 // 16-lane row (all rows and banks enabled, so every source is valid).

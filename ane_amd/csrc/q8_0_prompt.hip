@@ -55,6 +55,12 @@ struct Lay {
     static_assert(kLds <= 160 * 1024, "LDS");
 };
 
+// One workgroup per row group and token group; row groups in eights (XCDs).
+template <int TT>
+uint64_t grid_of(uint32_t N, uint32_t T) {
+    return ceil_to(((uint64_t)N + kRows - 1) / kRows, 8) * (((uint64_t)T + Lay<TT>::kTok - 1) / Lay<TT>::kTok);
+}
+
 // AL: every row starts 16-byte aligned (no lead-in bytes).
 template <int TT, bool AL>
 __global__ void __launch_bounds__(kWaves * 64)
@@ -247,13 +253,11 @@ int launch(uint32_t N, uint32_t nb, uint32_t T, const uint8_t* Wa, uint32_t off,
            const float* dxb, uint32_t Tp, float* y, hipStream_t s) {
     using L = Lay<TT>;
     const uint32_t rg = (N + kRows - 1) / kRows, tg = (T + L::kTok - 1) / L::kTok;
-    const uint64_t grid = ceil_to(rg, 8) * tg;
-    if (grid > 0x7fffffffull) return -1;
     const auto fn = k_q8_0_prompt<TT, AL>;
     if (hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)L::kLds) != hipSuccess)
         return ANE_ERR_HIP;
-    hipLaunchKernelGGL(fn, dim3((uint32_t)grid), dim3(kWaves * 64), L::kLds, s, N, nb, T, Wa, off, wrange, qxb, dxb, Tp,
+    hipLaunchKernelGGL(fn, dim3((uint32_t)grid_of<TT>(N, T)), dim3(kWaves * 64), L::kLds, s, N, nb, T, Wa, off, wrange, qxb, dxb, Tp,
                        tg, rg, y);
     ANE_HIP_CHECK_LAUNCH();
     return ANE_OK;
@@ -264,8 +268,8 @@ int launch(uint32_t N, uint32_t nb, uint32_t T, const uint8_t* Wa, uint32_t off,
 bool prompt_eligible(uint32_t N, uint32_t nb, uint32_t T, const void* W) {
     const uint64_t Tp = ((uint64_t)T + 15) & ~15ull;
     // 32-bit buffer offsets, with the windows' and tiles' over-read
-    return nb > 0 && (((uintptr_t)W) & 1) == 0 && (uint64_t)(N + kRows) * nb * 34 + 2048 < kOob &&
-           (nb + 1ull) * (Tp + 64) * 32 < kOob;
+    return nb > 0 && (((uintptr_t)W) & 1) == 0 && ((uint64_t)N + kRows) * nb * 34 + 2048 < kOob &&
+           (nb + 1ull) * (Tp + 64) * 32 < kOob && launch_fits(T <= 32 ? grid_of<1>(N, T) : grid_of<2>(N, T), kWaves * 64);
 }
 
 int prompt_mul_mat(uint32_t N, uint32_t nb, uint32_t T, const void* W, const void* qxb, const float* dxb, uint32_t Tp,

@@ -6,7 +6,7 @@
 
 namespace ane {
 
-// Whether the operands fit the kernel (W even, below 2 GiB).
+// Whether the operands (W even, below 2 GiB) and the launch fit the kernel.
 bool prompt_eligible(uint32_t N, uint32_t nb, uint32_t T, const void* W);
 // y[T x N] from activations already quantized in the form of k_q8_0_mmv
 // (q8_0_mmv.hpp, quantize_bt): qxb[b][Tp][32] int8, dxb[b][Tp] fp32, Tp = ceil16(T).

@@ -1,0 +1,27 @@
+"""The sizes at which a kernel's own launch or 32-bit arithmetic ends, on the CPU:
+the rules that leave such calls to another route (no GPU needed)."""
+import ctypes
+
+import pytest
+
+import ane_amd
+
+
+def rule(mangled, restype, *argtypes):
+    f = getattr(ane_amd.lib(), mangled)
+    f.restype, f.argtypes = restype, argtypes
+    return f
+
+
+@pytest.mark.parametrize("N,nb,T,fits", [
+    (4096, 128, 512, True), (1, 1, 5, True),
+    # weights of 2 GiB and more, and N + 64 past 2^32
+    (61_680_000, 1, 64, True), (63_161_284, 1, 64, False), ((1 << 32) - 64, 1, 5, False), ((1 << 32) - 1, 1, 5, False),
+    # 512 threads per 64 rows x 64 tokens (x 32 up to 32 tokens): 2^32 work items
+    (1 << 20, 1, 32704, True), (1 << 20, 1, 32768, False), ((1 << 20) + 64, 1, 32768, False),
+    (1 << 11, 1, 16_700_000, True), (1 << 12, 1, 16_700_000, False),
+])
+def test_prompt_kernel(N, nb, T, fits):
+    """ane::prompt_eligible (q8_0_prompt.hip)."""
+    f = rule("_ZN3ane15prompt_eligibleEjjjPKv", ctypes.c_bool, *[ctypes.c_uint32] * 3, ctypes.c_void_p)
+    assert f(N, nb, T, 0) == fits
