@@ -36,6 +36,12 @@ struct ane_ggml_backend {
 };
 
 namespace ane {
+
+uint64_t flat_ew_blocks(uint64_t n) {
+    const uint64_t wgs = (n / 4 + 511) / 512 + 1;
+    return launch_fits(wgs, 256) ? wgs : 0;
+}
+
 namespace {
 
 // rows x cols fp32, source rows `stride` bytes apart -> contiguous dst.
@@ -416,8 +422,8 @@ int rows_ew(ane_ggml_backend* be, const ane_ggml_tensor* d, const ane_ggml_tenso
         float* o = static_cast<float*>(d->data);
         const float* x = static_cast<const float*>(a->data);
         const float* y = b ? static_cast<const float*>(b->data) : nullptr;
-        const uint64_t n = ne0 * rows, wgs = (n / 4 + 511) / 512 + 1;
-        if ((!b || (same_shape(b, d) && contiguous(b))) && wgs <= 0x7fffffffull) {
+        const uint64_t n = ne0 * rows, wgs = flat_ew_blocks(n);
+        if ((!b || (same_shape(b, d) && contiguous(b))) && wgs) {
             hipLaunchKernelGGL(k_flat_ew<OP>, dim3((uint32_t)wgs), dim3(256), 0, be->stream, n, o, x, y, s);
             ANE_HIP_CHECK_LAUNCH();
             return ANE_OK;

@@ -43,6 +43,10 @@ __host__ __device__ inline uint64_t row_offset(const NodeRows& m, const RowIdx& 
     return row_repeat(i.i1, m.ne1) * m.nb1 + row_repeat(i.i2, m.ne2) * m.nb2 + row_repeat(i.i3, m.ne3) * m.nb3;
 }
 
+// Workgroups of the flat elementwise kernel (ggml_backend.hip) for n values; 0:
+// more than a launch holds (the row kernel, whose grid is bounded, takes them).
+uint64_t flat_ew_blocks(uint64_t n);
+
 // Row kernels in the reference handlers' arithmetic (decode_ref.hip), one
 // launch over `rows` rows of `dim` floats; every operand's innermost stride
 // is 4 bytes and its row offsets come from its NodeRows.

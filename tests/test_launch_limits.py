@@ -25,3 +25,13 @@ def test_prompt_kernel(N, nb, T, fits):
     """ane::prompt_eligible (q8_0_prompt.hip)."""
     f = rule("_ZN3ane15prompt_eligibleEjjjPKv", ctypes.c_bool, *[ctypes.c_uint32] * 3, ctypes.c_void_p)
     assert f(N, nb, T, 0) == fits
+
+
+@pytest.mark.parametrize("n,blocks", [(1, 1), (4, 2), (2048, 2), (2052, 3), (1 << 30, (1 << 19) + 1),
+                                      (((1 << 24) - 2) * 2048, (1 << 24) - 1), (((1 << 24) - 2) * 2048 + 4, 0),
+                                      (1 << 35, 0), (1 << 40, 0)])
+def test_flat_elementwise(n, blocks):
+    """ane::flat_ew_blocks (ggml_backend.hip): 256 threads a workgroup, 2^24
+    workgroups are one too many."""
+    f = rule("_ZN3ane14flat_ew_blocksEm", ctypes.c_uint64, ctypes.c_uint64)
+    assert f(n) == blocks
