@@ -41,6 +41,14 @@
 #include <type_traits>
 
 namespace ane {
+
+// The tile that many tokens take, 512 threads per 64 x 64 outputs.  The others
+// run below one such workgroup per CU, or for up to 32 tokens: 16 threads a row
+// at most, with N below 2^27 by the weights' 2 GiB.
+bool rmode_launch_fits(uint32_t N, uint32_t T) {
+    return T <= 32 || launch_fits(((uint64_t)N + 63) / 64 * (((uint64_t)T + 63) / 64), 512);
+}
+
 namespace {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -276,7 +284,6 @@ int launch(uint32_t N, uint32_t nb, uint32_t T, const float* x, const uint8_t* W
     using L = RLayout<F, RT, TT, WT, P>;
     const uint32_t tg = (T + L::kTok - 1) / L::kTok;
     const uint64_t grid = (uint64_t)((N + L::kRows - 1) / L::kRows) * tg;
-    if (grid > 0x7fffffffull) return -1;
     hipLaunchKernelGGL((k_rmode_mul_mat<F, RT, TT, WT, P>), dim3((uint32_t)grid), dim3(L::kThreads), 0, s, N, nb, T, x,
                        Wa, off, wrange, tg, y);
     ANE_HIP_CHECK_LAUNCH();
@@ -290,7 +297,7 @@ int run(uint32_t N, uint32_t nb, uint32_t T, const float* x, const void* W, floa
     // 32-bit buffer offsets: x, and the weights with the last window's over-read, below 2 GiB
     const uint64_t wbytes = off + (uint64_t)N * nb * F::kBytes;
     if (nb == 0 || (wp & 1) || (((uintptr_t)x) & 3) || wbytes + 2 * kMaxP * F::kBytes + 16 >= kOob ||
-        ((uint64_t)T + 64) * nb * 128 + 2 * kMaxP * 128 >= kOob)
+        ((uint64_t)T + 64) * nb * 128 + 2 * kMaxP * 128 >= kOob || !rmode_launch_fits(N, T))
         return -1;
     // Token t's y may take the place of an earlier token's x in the one launch
     // per token; here every token is read and written at once.

@@ -35,3 +35,13 @@ def test_flat_elementwise(n, blocks):
     workgroups are one too many."""
     f = rule("_ZN3ane14flat_ew_blocksEm", ctypes.c_uint64, ctypes.c_uint64)
     assert f(n) == blocks
+
+
+@pytest.mark.parametrize("N,T,fits", [(1, 2, True), (4096, 512, True), (119_000_000, 32, True),
+                                      (1 << 20, (1 << 15) - 64, True), (1 << 20, (1 << 15) - 63, False),
+                                      (1 << 15, 1 << 20, False), (119_000_000, 16_000_000, False)])
+def test_handlers_product(N, T, fits):
+    """ane::rmode_launch_fits (rmode_mul_mat.hip): 512 threads per 64 x 64 outputs
+    above 32 tokens."""
+    f = rule("_ZN3ane17rmode_launch_fitsEjj", ctypes.c_bool, *[ctypes.c_uint32] * 2)
+    assert f(N, T) == fits
