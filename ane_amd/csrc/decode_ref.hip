@@ -941,16 +941,18 @@ int softmax_node_launch(uint32_t dim, uint64_t rows, float scale, const uint8_t*
     return ANE_OK;
 }
 
+uint64_t rope_node_step(uint64_t rows, uint32_t pairs) {
+    uint64_t step = rows / 8 > 4096 ? rows / 8 : 4096;
+    if (step > rows) step = rows;
+    const uint64_t cap = ((1ull << 32) - 256) / pairs;  // whole workgroups, fewer than 2^24
+    return step > cap ? cap : step;
+}
+
 int rope_node_launch(uint32_t dim, uint64_t rows, float theta, const int32_t* pos, const uint8_t* in,
                      const NodeRows& src, uint8_t* out, const NodeRows& dst, hipStream_t s) {
     if (rows == 0 || dim < 2) return ANE_OK;
-    // 4096 rows per sweep, more where that would be over eight sweeps; at
-    // most 2^24 workgroups
     const uint32_t pairs = dim / 2;
-    uint64_t step = rows / 8 > 4096 ? rows / 8 : 4096;
-    if (step > rows) step = rows;
-    const uint64_t cap = (1ull << 32) / pairs;
-    if (step > cap) step = cap ? cap : 1;
+    const uint64_t step = rope_node_step(rows, pairs);
     hipLaunchKernelGGL(k_rope_node, dim3((uint32_t)((step * pairs + 255) / 256)), dim3(256), 0, s, dim, rows, step,
                        theta, pos, in, src, out, dst);
     ANE_HIP_CHECK_LAUNCH();

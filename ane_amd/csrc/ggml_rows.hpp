@@ -62,5 +62,8 @@ int softmax_node_launch(uint32_t dim, uint64_t rows, float scale, const uint8_t*
                         const uint8_t* mask, const NodeRows& msk, uint8_t* out, const NodeRows& dst, hipStream_t s);
 int rope_node_launch(uint32_t dim, uint64_t rows, float theta, const int32_t* pos, const uint8_t* in,
                      const NodeRows& src, uint8_t* out, const NodeRows& dst, hipStream_t s);
+// Rows that the RoPE kernel takes in one sweep, one thread per pair: 4096, more
+// where that would be over eight sweeps, at most what one launch holds.
+uint64_t rope_node_step(uint64_t rows, uint32_t pairs);
 
 }  // namespace ane

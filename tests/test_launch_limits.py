@@ -45,3 +45,13 @@ def test_handlers_product(N, T, fits):
     above 32 tokens."""
     f = rule("_ZN3ane17rmode_launch_fitsEjj", ctypes.c_bool, *[ctypes.c_uint32] * 2)
     assert f(N, T) == fits
+
+
+@pytest.mark.parametrize("rows,pairs,step", [(1, 64, 1), (4096, 64, 4096), (5000, 64, 4096), (40000, 64, 5000),
+                                             (1 << 29, 64, (1 << 26) - 4), (1 << 29, 1, 1 << 26), (7, 1 << 30, 3),
+                                             (2, (1 << 31) - 1, 1), (1 << 36, 1, (1 << 32) - 256)])
+def test_rope_sweep(rows, pairs, step):
+    """ane::rope_node_step (decode_ref.hip): a sweep stays below 2^32 threads."""
+    f = rule("_ZN3ane14rope_node_stepEmj", ctypes.c_uint64, ctypes.c_uint64, ctypes.c_uint32)
+    assert f(rows, pairs) == step
+    assert -(-step * pairs // 256) * 256 < 1 << 32
