@@ -194,10 +194,10 @@ constexpr uint32_t kPackT = 16;                     // groups and panels per wor
 constexpr uint32_t kPackStride = kPackT * 64 + 16;  // LDS bytes between panels
 
 __global__ void __launch_bounds__(kQThreads)
-k_pack_b(uint32_t K, uint32_t N, uint32_t G, uint32_t P, uint32_t pbase, const int8_t* __restrict__ src,
-         int8_t* __restrict__ dst) {
+k_pack_b(uint32_t K, uint32_t N, uint32_t G, uint32_t P, uint32_t gbase, uint32_t pbase,
+         const int8_t* __restrict__ src, int8_t* __restrict__ dst) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[kPackT * kPackStride];
-    const uint32_t g0 = blockIdx.x * kPackT, p0 = pbase + blockIdx.y * kPackT;
+    const uint32_t g0 = gbase + blockIdx.x * kPackT, p0 = pbase + blockIdx.y * kPackT;
     {
         const uint32_t p = threadIdx.x % kPackT, g = threadIdx.x / kPackT;
         const uint64_t col = 16ull * (p0 + p), k = 4ull * (g0 + g);
@@ -318,11 +318,15 @@ extern "C" int ane_hip_pack_b_i8(uint32_t K, uint32_t N, const int8_t* src, int8
     if (!src || !dst) return ANE_ERR_BAD_POINTER;
     const uint64_t gx = (G + kPackT - 1) / kPackT, gy = (P + kPackT - 1) / kPackT;
     if ((G * P + kQThreads - 1) / kQThreads > 0x7fffffffull) return ANE_ERR_INVALID_ARG;
-    // y-extent of a launch: 65535 workgroups of 16 panels
-    for (uint64_t y = 0; y < gy; y += 65535) {
-        const uint64_t ny = gy - y < 65535 ? gy - y : 65535;
-        hipLaunchKernelGGL(k_pack_b, dim3((uint32_t)gx, (uint32_t)ny), dim3(kQThreads), 0, (hipStream_t)stream, K, N,
-                           (uint32_t)G, (uint32_t)P, (uint32_t)(y * kPackT), src, dst);
+    // a launch holds 65535 workgroups of 16 panels in y and fewer than 2^24 (of 256
+    // threads) of 16 groups in x
+    constexpr uint64_t kMaxX = (1u << 24) - 1, kMaxY = 65535;
+    for (uint64_t y = 0; y < gy; y += kMaxY) {
+        for (uint64_t x = 0; x < gx; x += kMaxX) {
+            const uint64_t nx = gx - x < kMaxX ? gx - x : kMaxX, ny = gy - y < kMaxY ? gy - y : kMaxY;
+            hipLaunchKernelGGL(k_pack_b, dim3((uint32_t)nx, (uint32_t)ny), dim3(kQThreads), 0, (hipStream_t)stream, K,
+                               N, (uint32_t)G, (uint32_t)P, (uint32_t)(x * kPackT), (uint32_t)(y * kPackT), src, dst);
+        }
     }
     ANE_HIP_CHECK_LAUNCH();
     return ANE_OK;

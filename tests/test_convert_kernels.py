@@ -36,6 +36,23 @@ def test_pack_b_tiles(ane, oracle, K, N, offset):
         assert (got[:dst_off] == 77).all() and (got[dst_off + ref.size:] == 77).all()
 
 
+def test_pack_b_more_rows_than_a_launch(ane):
+    """2^30 + 5 rows of one column: more 64-row tiles than one launch holds (1 GiB
+    in, 16 GiB out, compared on the device)."""
+    import torch
+
+    K = (1 << 30) + 5
+    src = torch.randint(-128, 128, (K,), dtype=torch.int8, device="cuda")
+    out = torch.full((-(-K // 4) * 64,), 77, dtype=torch.int8, device="cuda")
+    ane.pack_b_i8(K, 1, src, out)
+    groups = out.view(torch.int32).view(-1, 16)  # a column's four rows per word
+    col = groups[:, 0].contiguous().view(torch.int8)
+    assert torch.equal(col[:K], src) and not col[K:].any()
+    assert not groups[:, 1:].any()
+    del src, out, groups, col
+    torch.cuda.empty_cache()
+
+
 # 1024 rows: one wave per row up to 2048 values; fewer rows or longer ones: a
 # workgroup per row, held in registers up to 8192 values
 @pytest.mark.parametrize("rows,cols", [(1024, 16), (1027, 100), (1025, 2048), (1024, 2064), (3, 8192), (2, 8200),
