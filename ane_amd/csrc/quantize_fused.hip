@@ -963,6 +963,9 @@ struct ResidentDevice {
     // the CUs and neither grid could pass its wait), so a launch on another
     // stream first waits for this event.
     hipEvent_t last = nullptr;
+    bool launched = false;  // the event was recorded
+    // The stream of the last such launch, or of the last uncaptured call that
+    // waited for it and took another route: work queued there runs after it.
     hipStream_t last_stream = nullptr;
     bool last_valid = false;
     uint32_t tag = 0;  // the last launch's tag (launches are numbered from 1)
@@ -1040,8 +1043,9 @@ bool launch_grid_wait(hipStream_t s, uint32_t ResidentDevice::*grid_of, bool eag
     // wait for work outside its graph, so under capture the route is taken
     // only on the stream of the previous launch (graph replays are ordered
     // by their caller).  An uncaptured call that the kernel fits but that takes
-    // another route is ordered the same way, so that it too makes its stream
-    // the one to capture on.
+    // another route waits for the previous launch in the same way, so that it
+    // too makes its stream the one to capture on; the event stays that
+    // launch's, so calls without a grid-wide wait never wait for each other.
     const bool other = d.last_valid && d.last_stream != s;
     if (capturing && other) return false;
     if (!capturing) {
@@ -1050,16 +1054,11 @@ bool launch_grid_wait(hipStream_t s, uint32_t ResidentDevice::*grid_of, bool eag
             d.last = nullptr;
             return false;
         }
-        if (other && hipStreamWaitEvent(s, d.last, 0) != hipSuccess) {
+        if (other && d.launched && hipStreamWaitEvent(s, d.last, 0) != hipSuccess) {
             (void)hipGetLastError();
             return false;
         }
         if (!eager) {
-            // recorded behind that wait, the event still covers the launch before
-            if ((other || !d.last_valid) && hipEventRecord(d.last, s) != hipSuccess) {
-                (void)hipGetLastError();
-                return false;
-            }
             d.last_stream = s;
             d.last_valid = true;
             return false;
@@ -1083,6 +1082,7 @@ bool launch_grid_wait(hipStream_t s, uint32_t ResidentDevice::*grid_of, bool eag
             *status = ANE_ERR_HIP;
             return true;
         }
+        d.launched = true;
         d.last_stream = s;
         d.last_valid = true;
     }

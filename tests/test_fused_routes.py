@@ -90,3 +90,51 @@ def test_capture_after_a_wait_on_another_stream(ane, oracle):
         ane.dense_fused_i8_status(ws, stream=s2)
         assert_same(host(C).reshape(M, N), want)
         assert int(host(ws[256 + 8192:256 + 8196]).view(np.uint32)[0]) > 0
+
+
+def test_two_pass_calls_do_not_wait_for_each_other(ane, oracle):
+    """With no grid-wide wait in flight, a two-pass call on one stream does not
+    run behind what another stream had queued before its own two-pass call."""
+    import torch
+
+    M, N, K = 256, 2048, 2048
+    A, B = data.gemm_inputs(M, N, K, seed=41)
+    want = oracle.dense_fused_i8(M, N, K, F32(1.0), True, A, B)
+    dA, dB, C = dev(A), dev(B), [torch.zeros(M * N, device="cuda") for _ in range(2)]
+    ws = [torch.empty(ane.dense_fused_i8_workspace_size(M, N, K), dtype=torch.uint8, device="cuda") for _ in range(2)]
+    x, y = torch.randn(8192, 8192, device="cuda"), torch.empty(8192, 8192, device="cuda")
+    busy, others = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(4)]
+
+    def call(i, s):
+        ane.dense_fused_i8(M, N, K, 1.0, True, dA, dB, C[i], workspace=ws[i], stream=s, check_wait=False)
+
+    def backlog():  # a few hundred milliseconds on `busy`
+        with torch.cuda.stream(busy):
+            for _ in range(30):
+                torch.mm(x, x, out=y)
+        return busy.record_event()
+
+    def independent(s):  # not on busy's hardware queue
+        end = backlog()
+        with torch.cuda.stream(s):
+            C[1].zero_()
+        s.record_event().synchronize()
+        free = not end.query()
+        torch.cuda.synchronize()
+        return free
+
+    for s in [busy] + others:
+        call(0, s)
+    backlog()
+    torch.cuda.synchronize()
+    s = next(s for s in others if independent(s))
+    call(1, others[0] if s is not others[0] else others[1])
+    torch.cuda.synchronize()
+    end = backlog()
+    call(0, busy)
+    call(1, s)
+    s.record_event().synchronize()
+    assert not end.query()
+    torch.cuda.synchronize()
+    for c in C:
+        assert_same(host(c).reshape(M, N), want)
