@@ -155,7 +155,7 @@ k_gemm_i8(GemmParams p) {
                     p.Craw[(uint64_t)i * p.ldc + j] = v;
                 } else if (p.ig) {
                     p.C[(uint64_t)i * p.ldc + j] =
-                        ig_out(p, v, ig_sum(p.igc, p.nsum, p.Nout, j), ig_sum(p.igr, p.nsum, p.Mout, i));
+                        ig_out(p, v, ig_sum<1>(p.igc, p.nsum, p.Nout, j), ig_sum<1>(p.igr, p.nsum, p.Mout, i));
                 } else {
                     float f = __fadd_rn(__fmul_rn((float)v, s), bj);
                     p.C[(uint64_t)i * p.ldc + j] = fmax_a(f, p.lo);

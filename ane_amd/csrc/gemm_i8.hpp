@@ -32,11 +32,25 @@ struct GemmParams {
     uint32_t nsum, corr;
 };
 
-// Sum of the partials of column or row x (n columns or rows in all); 0 without.
+// Partials per column or row, at most: each reader adds them up, so they pay
+// only while they are few (igemm.hip).
+constexpr uint32_t kIgParts = 16;
+
+// 128 * the sum of the partials of column or row x (n columns or rows in all); 0
+// without.  U loads are in flight at a time.
+template <uint32_t U = 8>
 __device__ __forceinline__ uint32_t ig_sum(const int32_t* part, uint32_t nsum, uint32_t n, uint32_t x) {
+    if (!part) return 0u;
+    const int32_t* c = part + (x < n ? x : n - 1);
+    if (nsum == 1) return 128u * (uint32_t)c[0];
     uint32_t t = 0;
-    if (part)
-        for (uint32_t p = 0; p < nsum; p++) t += (uint32_t)part[(uint64_t)p * n + (x < n ? x : n - 1)];
+    for (uint32_t p = 0; p < nsum; p += U) {
+        uint32_t v[U];
+#pragma unroll
+        for (uint32_t q = 0; q < U; q++) v[q] = (uint32_t)c[(uint64_t)(p + q < nsum ? p + q : p) * n];
+#pragma unroll
+        for (uint32_t q = 0; q < U; q++) t += p + q < nsum ? v[q] : 0u;
+    }
     return 128u * t;
 }
 __device__ __forceinline__ float ig_out(const GemmParams& p, int32_t acc, uint32_t col, uint32_t row) {

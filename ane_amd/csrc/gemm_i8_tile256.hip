@@ -326,15 +326,13 @@ ANE_TILE_KERNEL(GemmParams p, uint32_t tiles_m, uint32_t tiles_n) {
     const uint32_t rA = wr0 + (lane & 31);
     const uint32_t rB = wc0 + (lane & 31);
     const uint32_t chalf = lane >> 5;
-    // IG: the first kIgEarly partials of tile column tid, in flight during the K
-    // loop (summed before it they cost the loop's start: 17.2 -> 20.2 us at 1536 x
-    // 2048 x 2048)
-    constexpr uint32_t kIgEarly = 16;
-    uint32_t cpart[kIgEarly];
+    // IG: the partials of tile column tid, in flight during the K loop (summed
+    // before it they cost the loop's start: 17.2 -> 20.2 us at 1536 x 2048 x 2048)
+    uint32_t cpart[kIgParts];
     const uint32_t icol = col0 + tid < p.Nout ? col0 + tid : p.Nout - 1;
     if (IG)
 #pragma unroll
-        for (uint32_t q = 0; q < kIgEarly; q++)
+        for (uint32_t q = 0; q < kIgParts; q++)
             cpart[q] = p.igc && q < p.nsum ? (uint32_t)p.igc[(uint64_t)q * p.Nout + icol] : 0u;
 
     v16i acc[FM][FN];
@@ -449,9 +447,7 @@ ANE_TILE_KERNEL(GemmParams p, uint32_t tiles_m, uint32_t tiles_n) {
         if (tid < (uint32_t)TN) {
             uint32_t t = 0;
 #pragma unroll
-            for (uint32_t q = 0; q < kIgEarly; q++) t += cpart[q];
-            if (p.igc)
-                for (uint32_t q = kIgEarly; q < p.nsum; q++) t += (uint32_t)p.igc[(uint64_t)q * p.Nout + icol];
+            for (uint32_t q = 0; q < kIgParts; q++) t += cpart[q];
             w[tid] = 128u * t;
         }
         if (tid < (uint32_t)TM) w[TN + tid] = ig_sum(p.igr, p.nsum, p.Mout, row0 + tid);
@@ -561,6 +557,7 @@ int ANE_TILE_LAUNCH(const GemmParams& p, hipStream_t s, uint32_t ksplit) {
     const uint64_t total = (uint64_t)tiles_m * tiles_n;
     if (total > 0x7fffffffull || ksplit == 0 || ksplit > 65535) return ANE_ERR_INVALID_ARG;
     if (ksplit > 1 && !p.Craw) return ANE_ERR_INVALID_ARG;  // split K writes int32 planes
+    if (p.ig && p.nsum > kIgParts) return ANE_ERR_INVALID_ARG;
     const auto fn = p.ig ? ANE_TILE_KERNEL<true> : ANE_TILE_KERNEL<false>;
     hipLaunchKernelGGL(fn, dim3((uint32_t)total, ksplit), dim3(kThreads), 0, s, p, tiles_m, tiles_n);
     ANE_HIP_CHECK_LAUNCH();

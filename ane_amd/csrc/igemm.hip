@@ -259,10 +259,16 @@ extern "C" int ane_hip_cblas_igemm(int variant, int semantics, uint8_t flags, ui
         if (au || bu) {
             // Partial sums per k-tile in the int32 sums' place when the
             // contraction writes C itself and they fit there (and in the row
-            // and column sums after it); else one cleared sum per row.
+            // and column sums after it); else one cleared sum per row.  Not
+            // more than kIgParts of them (K <= 2048), which the readers add up:
+            // uint8 x uint8, partials without that bound and sums, 128 x 4096 x
+            // 8192 63.6 / 52 us, 300 x 300 x 8192 41.0 / 35.1, 1024 x 1024 x 16384
+            // 76.2 / 53.4; 128 x 4096 x 1024 13.9 / 15.8, 1536 x 2048 x 2048 21.1 /
+            // 22.6.  And not for the narrow products that k_gemm_i8 takes, which
+            // adds them up for every element (40000 x 16 x 2048 156 / 74).
             const uint32_t kt = (Ke + kTK - 1) / kTK;
             const uint64_t have = (uint64_t)M * N + M + N, need = (uint64_t)kt * ((au ? N : 0) + (bu ? M : 0));
-            const bool parts = !reads_c && need <= have;
+            const bool parts = !reads_c && need <= have && kt <= kIgParts && (M <= 128 || N >= 128);
             int32_t* const csum = parts ? w.acc : w.colsum;
             int32_t* const rsum = parts ? w.acc + (au ? (uint64_t)kt * N : 0) : w.rowsum;
             if (!parts) {
