@@ -290,6 +290,32 @@ int launch(uint32_t N, uint32_t nb, uint32_t T, const float* x, const uint8_t* W
     return ANE_OK;
 }
 
+// Two or three tokens on rows the streaming GEMV takes (16-byte aligned): one
+// launch here costs the same for 1 to 16 tokens, the GEMVs once per token, and
+// from more than one workgroup (16 rows) per CU on they stream the weights two to
+// four times as fast.  Where two or three of them are the faster ones, GEMVs /
+// this kernel, us:
+//  * Q4_0, two tokens, K > 1024 from two workgroups per CU (9216 x 4096 24.3 /
+//    28.4, 28672 x 8192 91 / 114; 8192 x 4096 20.3 / 19.0, 14336 x 1024 12.1 /
+//    12.0), K > 4096 from one (6144 x 14336 54.6 / 57.8);
+//  * Q8_0, two tokens, K <= 4096 (4128 x 4096 18.1 / 24.6, 28672 x 4096 61.6 /
+//    88.1), from two workgroups per CU for K <= 1024 (6144 x 1024 9.7 / 9.3, 14336 x
+//    1024 14.4 / 18.5); longer rows, whose GEMV keeps fewer waves per CU, up to one
+//    and a half workgroups for K <= 8192 (6144 x 8192 32.2 / 45.2) and from three
+//    (14336 x 11008 78.7 / 122, 20000 x 11264 138 / 153), not between, where the
+//    GEMV's last round of waves is nearly empty (8192 x 8192 54.6 / 45.5, 10000 x
+//    11008 99.7 / 92.1);
+//  * Q8_0, three tokens, K <= 4096 from eight workgroups per CU (65536 x 2048 87.7 /
+//    118; 28672 x 4096 92.2 / 88.3).
+bool gemvs_faster(bool q4, uint32_t N, uint32_t nb, uint32_t T, uint64_t cus) {
+    const uint64_t wgs = ((uint64_t)N + 15) / 16;
+    if (wgs <= cus) return false;
+    if (q4) return T == 2 && nb > (wgs > 2 * cus ? 32u : 128u);
+    if (T == 3) return nb <= 128 && wgs > 8 * cus;
+    if (nb <= 128) return nb > 32 || wgs > 2 * cus;
+    return wgs > 3 * cus || (nb <= 256 && 2 * wgs <= 3 * cus);
+}
+
 template <class F>
 int run(uint32_t N, uint32_t nb, uint32_t T, const float* x, const void* W, float* y, hipStream_t s) {
     const uintptr_t wp = reinterpret_cast<uintptr_t>(W);
@@ -310,6 +336,8 @@ int run(uint32_t N, uint32_t nb, uint32_t T, const float* x, const void* W, floa
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return ANE_ERR_HIP;
+    if (T <= 3 && off == 0 && nb % 8 == 0 && gemvs_faster(std::is_same<F, Q40Lane>::value, N, nb, T, (uint64_t)cus))
+        return -1;
     auto wgs = [&](uint32_t rows, uint32_t tok) {
         return (uint64_t)((N + rows - 1) / rows) * ((T + tok - 1) / tok);
     };

@@ -11,7 +11,7 @@ namespace ane {
 // Bit-identical to one ane_hip_q4_0_gemv / ane_hip_q8_0_gemv per token.
 // -1 (nothing queued) for a shape it does not take: no blocks, weights at an
 // odd address, operands of 2 GiB or more, y overlapping x, a launch that does
-// not fit.
+// not fit, two or three tokens that the GEMVs serve faster.
 int rmode_mul_mat(bool q4, uint32_t N, uint32_t K, uint32_t T, const float* x, const void* W, float* y,
                   hipStream_t s);
 // Whether N x T outputs fit one launch.

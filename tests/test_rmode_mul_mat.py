@@ -33,7 +33,10 @@ def want(oracle, q4, N, K, W, x):
 # (N, K, T): each tile shape of the dispatch (by rows and tokens), its edges,
 # and K of 1 to 5 blocks over the 4-block stages
 SHAPES = [(16, 32, 2), (1, 64, 3), (17, 128, 16), (33, 160, 17), (100, 416, 31), (300, 512, 33), (4096, 128, 64),
-          (8200, 96, 65), (2050, 256, 130), (9000, 160, 33), (16400, 64, 70)]
+          (8200, 96, 65), (2050, 256, 130), (9000, 160, 33), (16400, 64, 70),
+          # two and three tokens on aligned rows ((N + T) % 8 == 0), both sides of
+          # the rule that leaves them to the GEMVs (256 CUs)
+          (4094, 256, 2), (4110, 1280, 2), (4109, 1280, 3), (8206, 256, 2), (8206, 1280, 2), (33005, 256, 3)]
 
 
 @pytest.mark.parametrize("q4", [True, False])
