@@ -334,6 +334,19 @@ def test_dense_fused_parity(ane, oracle, M, N, K, relu, scale):
     assert_f32_identical(host(C).reshape(M, N), ref)
 
 
+def waited(ws):
+    """Whether the last quantize call on this workspace ran the one-launch
+    resident quantizer: its wait record counts the workgroups that met."""
+    return int(host(ws[256 + 8192: 256 + 8196]).view(np.uint32)[0]) > 0
+
+
+def fused_in_two_calls(ane, M, N, K, relu, A, B, C, ws, stream=None, check_wait=None):
+    """_quantize, which takes the resident quantizer from 12 MiB of operands
+    (an uncaptured whole call from 112 MiB), then _gemm."""
+    ane.dense_fused_i8_quantize(M, N, K, A, B, ws, stream=stream, check_wait=check_wait)
+    ane.dense_fused_i8_gemm(M, N, K, 1.0, relu, C, ws, stream=stream)
+
+
 _SPECIAL = [(c, *shape) for c in ("a_nan", "b_inf", "a_neg_inf", "a_zero", "b_tiny")
             for shape in ((129, 257, 1000), (256, 512, 2048), (256, 2048, 2048))]
 _SPECIAL += [("a_nan", 5000, 64, 4096), ("b_inf", 5000, 64, 4096), ("a_neg_inf", 5000, 64, 4096)]
@@ -345,11 +358,12 @@ def test_dense_fused_special_operands(ane, oracle, case, M, N, K):
     special-cases: a NaN or an infinity (NaN or infinite per-tensor scale),
     an all-zero tensor (the zero guard) and a tensor of denormals and signed
     zeros only (127 / amax overflows to +inf, so 0 * inf reaches the
-    quantizer).  256 x 2048 x 2048 (18 MiB of operands) takes the one-launch
-    resident quantizer, the others the two-pass one.  5000 x 64 x 4096 takes
-    the resident quantizer with A's share larger than LDS and registers hold
-    (its rest re-read after the B tiles on the exact pack4 route that a
-    non-finite scale selects); the NaN sits in that re-read rest."""
+    quantizer).  The whole call through stream_exec takes the two-pass
+    quantizer (below 112 MiB of operands).  _quantize and _gemm take the
+    one-launch resident one for 256 x 2048 x 2048 (18 MiB), and for 5000 x 64
+    x 4096 with A's share larger than LDS and registers hold (its rest
+    re-read after the B tiles on the exact pack4 route that a non-finite
+    scale selects; the NaN sits in that re-read rest)."""
     import torch
 
     A, B = data.gemm_inputs(M, N, K, seed=M + K)
@@ -372,7 +386,13 @@ def test_dense_fused_special_operands(ane, oracle, case, M, N, K):
     finally:
         oracle.set_threads(1)
     C = zeros(M * N, torch.float32)
-    ane.stream_exec(ane.rec_dense_fused_i8(M, N, K, 1.0, True, dev(A), dev(B), C))
+    dA, dB = dev(A), dev(B)
+    ane.stream_exec(ane.rec_dense_fused_i8(M, N, K, 1.0, True, dA, dB, C))
+    assert_f32_identical(host(C).reshape(M, N), ref)
+    C.zero_()
+    ws = torch.empty(ane.dense_fused_i8_workspace_size(M, N, K), dtype=torch.uint8, device="cuda")
+    fused_in_two_calls(ane, M, N, K, True, dA, dB, C, ws)
+    assert waited(ws) == (K % 128 == 0 and N % 64 == 0 and 4 * (M * K + K * N) >= 12 << 20)
     assert_f32_identical(host(C).reshape(M, N), ref)
 
 
@@ -441,13 +461,16 @@ def test_dense_fused_few_tile_special_operands(ane, oracle, case):
     assert_f32_identical(host(C).reshape(M, N), ref)
 
 
-@pytest.mark.parametrize("M,N,K", [(256, 2048, 2048), (5000, 64, 4096), (777, 2048, 4096), (64, 2048, 2048)])
+@pytest.mark.parametrize("M,N,K", [(256, 2048, 2048), (5000, 64, 4096), (777, 2048, 4096), (64, 2048, 2048),
+                                   (7168, 64, 4096)])
 def test_dense_fused_resident_quantizer_shapes(ane, oracle, M, N, K):
     """Shapes on the one-launch resident quantizer (K % 128 == 0, N % 64 == 0,
     at least 12 MiB of operands): a workgroup's share of A all in LDS
     (256, 777 and 64 rows; 777 rows give every workgroup a ragged share), and
     past LDS into registers and the batched re-read (5000 x 4096: 20,000
-    float4 per workgroup, the last batch ragged)."""
+    float4 per workgroup, the last batch ragged).  _quantize and _gemm take
+    it for all of them, the whole call through stream_exec for the last
+    (113 MiB: uncaptured, from 112 MiB up)."""
     import torch
 
     A, B = data.gemm_inputs(M, N, K, seed=M + 3 * N + K)
@@ -457,8 +480,18 @@ def test_dense_fused_resident_quantizer_shapes(ane, oracle, M, N, K):
     finally:
         oracle.set_threads(1)
     C = zeros(M * N, torch.float32)
-    ane.stream_exec(ane.rec_dense_fused_i8(M, N, K, 1.0, False, dev(A), dev(B), C))
+    dA, dB = dev(A), dev(B)
+    ane.stream_exec(ane.rec_dense_fused_i8(M, N, K, 1.0, False, dA, dB, C))
     assert_f32_identical(host(C).reshape(M, N), ref)
+    ws = torch.empty(ane.dense_fused_i8_workspace_size(M, N, K), dtype=torch.uint8, device="cuda")
+    for whole in (True, False):
+        C.zero_()
+        if whole:
+            ane.dense_fused_i8(M, N, K, 1.0, False, dA, dB, C, workspace=ws)
+        else:
+            fused_in_two_calls(ane, M, N, K, False, dA, dB, C, ws)
+        assert waited(ws) == (not whole or 4 * (M * K + K * N) >= 112 << 20)
+        assert_f32_identical(host(C).reshape(M, N), ref)
 
 
 @pytest.mark.parametrize("M,N,K", [(256, 2048, 2048), (1, 4096, 4096), (5000, 64, 4096), (300, 700, 333)])
@@ -580,11 +613,12 @@ def test_dense_fused_strip_special_operands(ane, oracle, case):
     assert_f32_identical(host(C).reshape(M, N), ref)
 
 
-@pytest.mark.parametrize("M,N,K", [(256, 2048, 2048), (8, 4096, 4096)])
+@pytest.mark.parametrize("M,N,K", [(7168, 64, 4096), (8, 4096, 4096), (256, 2048, 2048)])
 def test_dense_fused_grid_wait_limit(ane, oracle, M, N, K):
-    """The bounded grid-wide wait of the resident quantizer (256 x 2048 x
-    2048) and of the strip route (8 x 4096 x 4096), forced from the host
-    to a one-tick limit: every workgroup still finishes, and a launch whose
+    """The bounded grid-wide wait of the resident quantizer (7168 x 64 x 4096,
+    whole calls; 256 x 2048 x 2048, _quantize and _gemm, whose whole
+    uncaptured call has no wait) and of the strip route (8 x 4096 x 4096),
+    forced from the host to a one-tick limit: every workgroup still finishes, and a launch whose
     workgroups gave up is reported (C is then not valid) by stream_exec, by
     the kernel ABI's wait record (ane_hip_dense_fused_i8_status) and by the
     Python wrapper, each with ANE_ERR_GRID_WAIT; one that did not is exact.
@@ -604,6 +638,21 @@ def test_dense_fused_grid_wait_limit(ane, oracle, M, N, K):
     ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
     stream = ane._stream_handle(None)
     grid_wait = 9  # ANE_ERR_GRID_WAIT
+    split = M == 256
+
+    def abi():
+        if not split:
+            return lib.ane_hip_dense_fused_i8(M, N, K, 1.0, 1, ane._p(dA), ane._p(dB), ane._p(C), 0, ane._p(ws), wsb,
+                                              stream)
+        st = lib.ane_hip_dense_fused_i8_quantize(M, N, K, ane._p(dA), ane._p(dB), 0, ane._p(ws), wsb, stream)
+        return st or lib.ane_hip_dense_fused_i8_gemm(M, N, K, 1.0, 1, ane._p(C), ane._p(ws), wsb, stream)
+
+    def wrapped():
+        if split:
+            fused_in_two_calls(ane, M, N, K, True, dA, dB, C, ws)
+        else:
+            ane.dense_fused_i8(M, N, K, 1.0, True, dA, dB, C, workspace=ws)
+
     try:
         lib.ane_hip_set_grid_wait_limit(1)
         # opcode boundary
@@ -615,8 +664,8 @@ def test_dense_fused_grid_wait_limit(ane, oracle, M, N, K):
             assert_f32_identical(host(C).reshape(M, N), ref)
         # kernel ABI: the wait record in the caller's workspace
         C.zero_()
-        assert lib.ane_hip_dense_fused_i8(M, N, K, 1.0, 1, ane._p(dA), ane._p(dB), ane._p(C), 0, ane._p(ws),
-                                          wsb, stream) == 0
+        assert abi() == 0
+        assert waited(ws)
         st = lib.ane_hip_dense_fused_i8_status(ane._p(ws), stream)
         assert st in (0, grid_wait)
         if st == 0:
@@ -625,7 +674,7 @@ def test_dense_fused_grid_wait_limit(ane, oracle, M, N, K):
         # Python wrapper: checks after the call by default
         C.zero_()
         try:
-            ane.dense_fused_i8(M, N, K, 1.0, True, dA, dB, C, workspace=ws)
+            wrapped()
         except ane.AneError as e:
             assert e.status == grid_wait
         else:
@@ -638,11 +687,10 @@ def test_dense_fused_grid_wait_limit(ane, oracle, M, N, K):
         if how == "stream_exec":
             ane.stream_exec(ane.rec_dense_fused_i8(M, N, K, 1.0, True, dA, dB, C))
         elif how == "abi":
-            assert lib.ane_hip_dense_fused_i8(M, N, K, 1.0, 1, ane._p(dA), ane._p(dB), ane._p(C), 0, ane._p(ws),
-                                              wsb, stream) == 0
+            assert abi() == 0
             assert lib.ane_hip_dense_fused_i8_status(ane._p(ws), stream) == 0
         else:
-            ane.dense_fused_i8(M, N, K, 1.0, True, dA, dB, C, workspace=ws)
+            wrapped()
         assert lib.ane_hip_grid_wait_status(stream) == 0
         assert_f32_identical(host(C).reshape(M, N), ref)
 
@@ -661,10 +709,11 @@ def test_dense_fused_status_unwritten_workspace(ane):
     assert lib.ane_hip_dense_fused_i8_status(0, stream) == 8
 
 
-@pytest.mark.parametrize("M,N,K", [(256, 2048, 2048), (16, 4096, 4096)])
+@pytest.mark.parametrize("M,N,K", [(7168, 64, 4096), (16, 4096, 4096), (256, 2048, 2048)])
 def test_dense_fused_resident_two_streams(ane, oracle, M, N, K):
     """Two dense_fused_i8 calls with a grid-wide wait (the resident
-    quantizer, 256 x 2048 x 2048; the strip route, 16 x 4096 x 4096) issued
+    quantizer, 7168 x 64 x 4096 and, as _quantize and _gemm, 256 x 2048 x
+    2048; the strip route, 16 x 4096 x 4096) issued
     back to back on two streams with nothing between them: each grid needs
     every CU, so the library orders the second launch after the first (a
     stream-event wait); both results are exact and no wait gives up."""
@@ -683,8 +732,12 @@ def test_dense_fused_resident_two_streams(ane, oracle, M, N, K):
     torch.cuda.synchronize()
     for rep in range(3):
         for (dA, dB, C, ws), st in zip(bufs, streams):
-            ane.dense_fused_i8(M, N, K, 1.0, True, dA, dB, C, workspace=ws, stream=st, check_wait=False)
+            if M == 256:
+                fused_in_two_calls(ane, M, N, K, True, dA, dB, C, ws, stream=st, check_wait=False)
+            else:
+                ane.dense_fused_i8(M, N, K, 1.0, True, dA, dB, C, workspace=ws, stream=st, check_wait=False)
         for (dA, dB, C, ws), st in zip(bufs, streams):
+            assert waited(ws)
             ane.dense_fused_i8_status(ws, stream=st)
             assert ane.lib().ane_hip_grid_wait_status(ane._stream_handle(st)) == 0
         for (dA, dB, C, ws), ref in zip(bufs, refs):
