@@ -23,9 +23,13 @@ def run(ane, N, K, T, W, x, offset=0):
 
 
 # K: whole stages of 512, part stages, under one stage, odd block counts
-# (rows that are only 2-byte aligned); N and T around the tile edges
+# (rows that are only 2-byte aligned); N and T around the tile edges.  Aligned
+# rows (offset 0) with several stages: 136 blocks (the last stage half full) and
+# 64 blocks on 195 workgroups; the other whole-stage shapes are too few
+# workgroups for this kernel at offset 0
 @pytest.mark.parametrize("N,K,T", [(64, 512, 64), (65, 1024, 65), (63, 544, 33), (1, 32, 70), (130, 480, 100),
-                                   (200, 4128, 31), (64, 96, 5), (300, 2080, 129), (1000, 11008, 17), (7, 160, 200)])
+                                   (200, 4128, 31), (64, 96, 5), (300, 2080, 129), (1000, 11008, 17), (7, 160, 200),
+                                   (200, 4352, 100), (100, 4352, 20), (4100, 2048, 130)])
 @pytest.mark.parametrize("offset", [0, 6])
 def test_shapes(ane, oracle, N, K, T, offset):
     W = data.q8_0_weights(N, K, seed=N + K)
@@ -33,7 +37,7 @@ def test_shapes(ane, oracle, N, K, T, offset):
     assert_same(run(ane, N, K, T, W, x, offset), oracle.q8_0_mul_mat_g(N, K, T, x, W))
 
 
-@pytest.mark.parametrize("K", [544, 1024])
+@pytest.mark.parametrize("K", [544, 1024, 4352])
 def test_special_scales(ane, oracle, K):
     N, T = 70, 72
     W = data.q8_0_weights(N, K, seed=3).reshape(N, K // 32, 34).copy()
