@@ -1,12 +1,13 @@
-// gemm_i8_skinny.hip -- the int8 contraction for few rows (M <= 128): the
-// small-M end of dense_fused_i8's M sweep and gemm_s8_i32.  Output tiles of
+// gemm_i8_skinny.hip -- the int8 contraction for few rows (M <= 128, and more in
+// 64-row groups while that is at most one workgroup per CU): the small-M end of
+// dense_fused_i8's M sweep, dense_i8 / dense_u8s8, cblas_igemm and gemm_s8_i32.  Output tiles of
 // 128 x 128 would give 4096 columns only 32 workgroups, so the operand that
 // matters, Bt (N x Kp), would stream through 32 CUs.
 //
 // Design (gfx950):
 //  * One workgroup per 16 output columns: ceil(N/16) workgroups of 4 waves
 //    (256 for N = 4096).  The workgroup holds every output row (up to 8
-//    16-row blocks, MB) of its columns.
+//    16-row blocks, MB) of its columns, or 64 of them above 128 rows.
 //  * K advances in 128-byte steps; wave w takes steps w, w+4, w+8, ... (the
 //    four waves together read each Bt row front to back).  A step is two
 //    v_mfma_i32_16x16x64_i8 per row block: lane l loads the 32 contiguous

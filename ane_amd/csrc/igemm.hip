@@ -28,11 +28,12 @@
 //   16384 * Ke            (both)
 // which is exact modulo 2^32, like the handler's own wrapping sums.  Each tile
 // writes its rows' partial sums, added up in the epilogue (no atomics, nothing
-// to clear).  Signed operands that are already K-contiguous rows (A without
-// transA, B with transB) with 16-byte aligned rows that C does not overlap skip
-// the pre-pass: the contraction reads them in place.  With beta = 0 the contraction writes C
+// to clear), or for long K adds them into one cleared sum per row.  Signed
+// operands that are already K-contiguous rows (A without transA, B with transB)
+// with 16-byte aligned rows that C does not overlap skip the pre-pass: the
+// contraction reads them in place.  With beta = 0 the contraction writes C
 // itself; otherwise it leaves int32 sums and k_igemm_epilogue reads C.
-// Measured, 1536 x 2048 x 2048 uint8 x int8, both row-major: 27.4 -> 17.6 us
+// Measured, 1536 x 2048 x 2048 uint8 x int8, both row-major: 27.4 -> 17.3 us
 // (byte loads into 64 x 64 tiles with atomic row sums, a fill, two gathers and
 // a separate epilogue pass over 12.6 MB of sums before).
 #include "gemm_i8.hpp"

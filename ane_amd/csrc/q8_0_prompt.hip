@@ -28,9 +28,12 @@
 // XCD, whose L2 then reads those weights once for all token groups.
 //
 // Measured with the quantizer, before (k_q8_0_mmt / k_q8_0_mma, 16 x 16 tiles)
-// and now: 14336 x 4096 at 512 tokens 188 -> 145 us (2.4 us per stage of a
-// workgroup, of which the VALU's converts and fmas take about 1.2), 4096 x
-// 4096 100 -> 42, 28672 x 4096 310 -> 279, 4096 x 14336 at 256 tokens 95 -> 63.
+// and now: 14336 x 4096 at 512 tokens 188 -> 143 us (2.4 us per stage of a
+// workgroup, of which the VALU's converts and fmas take about 1.2: the two MFMAs
+// of a tile issue back to back, so the wave reaches that work only after the
+// passes of the first), 4096 x 4096 100 -> 42, 28672 x 4096 310 -> 279, 4096 x 14336
+// at 256 tokens 95 -> 63.  The 64-token forms use all 256 VGPRs and spill three or
+// four.
 #include "common.hpp"
 #include "q8_0_prompt.hpp"
 

@@ -20,8 +20,8 @@
 // never leaves the pointer's 16-byte granule at the front and reads zeros
 // past the matrix's last dword), two stages in flight in registers, each
 // stage written to the group's own LDS window and decoded from there with
-// byte reads.  x is staged in LDS in chunks of 4096 values shared by the
-// workgroup's rows.
+// byte reads.  x is staged in LDS in chunks of 4096 values (2048 at
+// 8 rows) shared by the workgroup's rows.
 #include "../../include/ane_hip.h"
 #include "common.hpp"
 #include "qformats.hpp"

@@ -16,10 +16,12 @@
 // a loop of this instruction reaches, with the weights' decode (about five
 // VALU operations per weight, once per 16*TT tokens) on the VALU beside it;
 // below that, the barrier and first reads of each stage with two waves per
-// SIMD.  Measured at 4096 x 4096 Q4_0, before (one GEMV launch per token,
-// decoding every weight again with the fmas on the VALU) and now: 2 tokens
-// 17.9 -> 13.0 us, 16 144 -> 13.8, 64 580 -> 32, 128 1158 -> 55 (78 TFLOP/s),
-// 512 4621 -> 182 (94 TFLOP/s); one token stays on the GEMV (9.2 us).
+// SIMD.  Measured at 4096 x 4096 Q4_0 (a call among many), before (one GEMV
+// launch per token, decoding every weight again with the fmas on the VALU) and
+// now: 2 tokens 17.9 -> 13.0 us, 16 144 -> 13.5, 64 579 -> 32.2, 128 1158 -> 49.7
+// (86 TFLOP/s), 512 4614 -> 182 (94 TFLOP/s); one token stays on the GEMV (9.2
+// us), and two or three over many rows do (gemvs_faster).  A kernel trace of a
+// dozen passes shows longer ones: 14.6, 36.1, 56.5 and 210 us for 16 to 512 tokens.
 //
 // Work split: a workgroup takes RT*16 rows x WT*TT*16 tokens with 4 x WT
 // waves.  Wave j of a token group runs chains 4j .. 4j+3 of all its

@@ -173,11 +173,18 @@ int ane_hip_dense_fused_i8(int32_t M, int32_t N, int32_t K, float scale,
  * follows applies to both.
  * Outside stream capture it is a cooperative launch: the runtime starts it
  * only with every workgroup resident, or refuses it and the two-pass route
- * (no wait) runs instead.  Under capture it is a plain launch.  Two such
+ * (no wait) runs instead.  Such a launch costs the stream 15-20 us more, so
+ * there ane_hip_dense_fused_i8 takes the quantizer from 112 MiB of operands
+ * only (the two-pass route below; the same bits); ..._quantize takes it from
+ * 12 MiB, and so does a whole call under capture, as a plain launch.  Two such
  * launches must not run at once on one device (each needs every CU): calls
  * on different streams are ordered by the library (a call waits for the
- * previous call's launch), and under capture the route is taken only on the
- * stream of the previous call.  Replays of captured graphs are not ordered
+ * last such launch), and under capture the route is taken only on the
+ * stream of the previous call whose shape the kernel fits.  An uncaptured
+ * call of such a shape that runs the two-pass route counts as that too: it
+ * waits for the last such launch if that was on another stream (not for what
+ * was queued there after it), and captures on its stream then keep the wait.
+ * Replays of captured graphs are not ordered
  * by the library: a replay that overlaps another replay or an eager call on
  * another stream makes the waits of both either time out or count each
  * other's arrivals.  Neither is silent: the wait is bounded (2 s by
